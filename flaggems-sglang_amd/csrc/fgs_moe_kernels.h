@@ -169,12 +169,12 @@ int launch_gemm2_direct(int dt, const GemmParams& p, int kw, hipStream_t stream)
 int launch_gemm2_pair(int dt, const GemmParams& p, int kw, hipStream_t stream);
 
 // LDS-tiled MFMA kernels (bf16, fp8, int8): configuration per element type
-// and rows-per-expert regime, its row block, n_out granularity, launch.
+// and rows-per-expert regime, its row block, launch. n_out is a multiple of
+// 128 (GEMM2's 256-column tiles may end in a half tile).
 constexpr int kTiledConfigs = 5;  // row blocks 256, 128, 64, 32, 160
 int tiled_config_supported(int dt, int cfg);
 int tiled_config_for(int dt, double rows_per_expert, int num_experts);
 int tiled_block_m(int cfg);
-int tiled_n_align(bool gemm1);
 int launch_gemm_tiled(int dt, int cfg, bool gemm1, const GemmParams& p,
                       int row_blocks, hipStream_t stream);
 // The tile plan the launch of launch_gemm_tiled(dt, cfg, gemm1, p,

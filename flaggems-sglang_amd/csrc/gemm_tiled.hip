@@ -153,6 +153,7 @@ __device__ __forceinline__ void tiled_tile(const GemmParams& p, const int rb_id,
   static_assert(STAGES >= 2 && (STAGES - 1) * NL < 64, "stages");
   static_assert(RB >= 1 && CB >= 1 && KK >= 1, "wave tile");
   static_assert(!GEMM1 || CB % 2 == 0, "gate/up pairing");
+  static_assert(128 % WCOLS == 0, "a wave's columns inside a 128-column block");
   static_assert(tiled_ring_bytes<DT, C, COMPACT>() <= 160 * 1024, "gfx950 LDS is 160 KiB");
   // a compact ring holds whole per-wave activation load groups
   static_assert(!COMPACT || C::BMA % (NLA * C::LR) == 0, "compact ring rows");
@@ -214,7 +215,8 @@ __device__ __forceinline__ void tiled_tile(const GemmParams& p, const int rb_id,
       const int ncol = tile_n * (BNR / 2) + wc * HALF + in % HALF;
       wrow = (in >= HALF ? p.n_out : 0) + ncol;
     } else {
-      wrow = static_cast<int64_t>(tile_n) * BNR + j;
+      // (a last tile of half the columns: the other half reads the last row)
+      wrow = min(static_cast<int64_t>(tile_n) * BNR + j, p.n_out - 1);
     }
     b_src[i] = p.w + (wbase + wrow) * row_bytes + chunk_pos<C>(j, lchunk) * 16;
   }
@@ -246,7 +248,7 @@ __device__ __forceinline__ void tiled_tile(const GemmParams& p, const int rb_id,
       if (slot < BM + (GEMM1 ? 2 : BNR / 128)) {
         const int b = slot - BM;
         wb = GEMM1 ? (b ? p.n_out / 128 : 0) + tile_n * (BNR / 2) / 128
-                   : static_cast<int64_t>(tile_n) * (BNR / 128) + b;
+                   : min(static_cast<int64_t>(tile_n) * (BNR / 128) + b, p.n_out / 128 - 1);
       }
       sc_src = p.w_scale + (wblk0 + wb) * kblocks;
     }
@@ -387,6 +389,11 @@ __device__ __forceinline__ void tiled_tile(const GemmParams& p, const int rb_id,
   int nlive = 0;
 #pragma unroll
   for (int i = 0; i < RB; ++i) nlive += first_sid[i] < p.numel ? 1 : 0;
+  // GEMM2 outputs of an odd multiple of 128 columns end in a tile of half
+  // the columns: a wave whose columns lie past the output (its WCOLS divide
+  // 128: all of them or none) loads for the others but multiplies nothing
+  const bool no_cols = !GEMM1 && static_cast<int64_t>(tile_n) * BNR + wn * WCOLS >= p.n_out;
+  if (no_cols) nlive = 0;
 
   Frag fa[2][RB], fb[2][CB];
   auto main_loop = [&](auto nlive_c, auto a_on_c) {
@@ -554,6 +561,7 @@ __device__ __forceinline__ void tiled_tile(const GemmParams& p, const int rb_id,
   constexpr int REGION = (STAGE / NW) & ~15;
   const int fslot = KT >= 2 ? (KT - 2) % STAGES : 0;
   if (KT < 2) wave_barrier_all();
+  if (no_cols) return;  // (no barrier of the workgroup follows)
   uint8_t* stg = lds + fslot * STAGE + wave * REGION;
   // orders this wave's staging writes before its reads (and the reads
   // before the next pass's writes)
@@ -862,7 +870,7 @@ __global__ __launch_bounds__(C::NW * 64, 1) void moe_gemm_tiled_kernel(
   constexpr int BM = C::BM, BNR = C::BNR;
 
   constexpr int N_PER_TILE = GEMM1 ? BNR / 2 : BNR;
-  const int n_ct = static_cast<int>(p.n_out / N_PER_TILE);
+  const int n_ct = static_cast<int>((p.n_out + N_PER_TILE - 1) / N_PER_TILE);
   int rb_id, tile_n;
   if (!tile_of(blockIdx.x, gridDim.x, p.row_blocks * p.ksplit, n_ct, p.group_m,
                p.group_n, &rb_id, &tile_n))
@@ -935,7 +943,8 @@ static int launch_tiled(const GemmParams& p, int row_blocks, hipStream_t stream)
   if (attr != hipSuccess)
     return fail(FGS_ELAUNCH, std::string("tiled GEMM LDS opt-in: ") +
                                  hipGetErrorString(attr));
-  const int tiles_n = static_cast<int>(GEMM1 ? p.n_out / (C::BNR / 2) : p.n_out / C::BNR);
+  constexpr int kCols = GEMM1 ? C::BNR / 2 : C::BNR;
+  const int tiles_n = static_cast<int>((p.n_out + kCols - 1) / kCols);
   GemmParams q = p;
   q.row_blocks = row_blocks;
   set_topk_magic(&q);
@@ -1019,10 +1028,6 @@ int tiled_config_for(int dt, double rows_per_expert, int num_experts) {
 }
 
 int tiled_block_m(int cfg) { return kTileRows[cfg]; }
-
-// n_out granularity the tiled kernels need: GEMM1 output cols per tile,
-// GEMM2 output cols per tile (every configuration uses BNR = 256).
-int tiled_n_align(bool gemm1) { return gemm1 ? 128 : 256; }
 
 template <int DT, class C>
 static int launch_cfg(bool gemm1, const GemmParams& p, int row_blocks,

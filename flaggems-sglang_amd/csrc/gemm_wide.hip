@@ -273,7 +273,7 @@ __global__ __launch_bounds__(C::NW * 64, 1) void moe_gemm_wide_kernel(const Gemm
   const int64_t row_bytes = p.kdim * ESZ;
   const int npp = __builtin_amdgcn_readfirstlane(p.num_post_pad[0]);
   constexpr int N_PER_TILE = GEMM1 ? BNR / 2 : BNR;
-  const int n_ct = static_cast<int>(p.n_out / N_PER_TILE);
+  const int n_ct = static_cast<int>((p.n_out + N_PER_TILE - 1) / N_PER_TILE);
   const int KT_all = static_cast<int>(row_bytes / SK);
 
   // ---- tile walk. The live tiles -- row blocks below
@@ -360,6 +360,8 @@ __global__ __launch_bounds__(C::NW * 64, 1) void moe_gemm_wide_kernel(const Gemm
         const int in = j % WCOLS;
         wrow = (in >= HALF ? p.n_out : 0) + t.ct * (BNR / 2) + wc * HALF + in % HALF;
       } else {
+        // (rows past an output that ends in half a tile lie past the
+        // expert's weight resource: their loads fetch nothing)
         wrow = static_cast<int64_t>(t.ct) * BNR + j;
       }
       s.vb[i] = static_cast<uint32_t>(wrow * row_bytes + wide_chunk<C>(j, lchunk) * 16);
@@ -476,6 +478,10 @@ __global__ __launch_bounds__(C::NW * 64, 1) void moe_gemm_wide_kernel(const Gemm
 #pragma unroll
   for (int i = 0; i < RB; ++i) nlive += first_sid[i] < p.numel ? 1 : 0;
   nlive = __builtin_amdgcn_readfirstlane(nlive);
+  // GEMM2 outputs of an odd multiple of 128 columns end in a tile of half
+  // the columns: the waves of the other half load but multiply and store
+  // nothing
+  if (!GEMM1 && static_cast<int64_t>(cur.ct) * BNR + wn * WCOLS >= p.n_out) nlive = 0;
 
   // The tile (accumulators, k loop, epilogue) is instantiated per count of
   // live 32-row blocks: all-pad blocks (the tail of an expert's last block)
@@ -615,7 +621,7 @@ __global__ __launch_bounds__(C::NW * 64, 1) void moe_gemm_wide_kernel(const Gemm
     // whole row segments, 16 bytes per lane. Chunks (16 bytes) of a staged
     // row are XOR-swizzled by the row so the column-major writes spread over
     // the banks.
-    {
+    if constexpr (NLIVE > 0) {
       const int ks = cur.ks;
       const int64_t wbase = static_cast<int64_t>(cur.e) * p.nrows_w;
 
@@ -896,7 +902,7 @@ __global__ __launch_bounds__(256) void moe_wide_tail_fixup_kernel(const GemmPara
   const int t = (blockIdx.x / 8) % 32;
   const int rblk = blockIdx.x / (8 * 32);
   const int npp = p.num_post_pad[0];
-  const int n_ct = static_cast<int>(p.n_out / BNR);
+  const int n_ct = static_cast<int>((p.n_out + BNR - 1) / BNR);
   const int total = npp / BM * n_ct;  // ksplit is 1 with a tail split
   const WideRange range = wide_range(p, total, xcd);
   const WideTail tail = wide_tail(range.lo, range.hi, true, static_cast<int>(p.kdim * ESZ / SK));
@@ -904,6 +910,7 @@ __global__ __launch_bounds__(256) void moe_wide_tail_fixup_kernel(const GemmPara
   int rb, ct;
   if (!wide_walk(range.lo, range.hi, n_ct, p.group_n, 32 * tail.R + t, &rb, &ct)) return;
   const int lane = threadIdx.x & 63;
+  if (static_cast<int64_t>(ct) * BNR + lane * 4 >= p.n_out) return;  // half a tile's columns
   const int slot0 = xcd * 32 + t * tail.S;
   // a wave's 8 rows in two batches of 4, every piece of a batch's rows in
   // flight at once (the reads, not the adds, set this kernel's time)
@@ -969,7 +976,7 @@ bool wide_supported(int dt, bool gemm1, const GemmParams& p) {
   if (row_bytes % C::SK != 0) return false;
   const int ks = std::max(1, gemm1 ? 1 : p.ksplit);
   if (row_bytes / C::SK < 2 * ks) return false;  // the prologue loads two stages
-  if (p.n_out % (gemm1 ? C::BNR / 2 : C::BNR) != 0) return false;
+  if (p.n_out % 128 != 0) return false;  // whole GEMM1 tiles; whole or half GEMM2 tiles
   constexpr int64_t kMax = (int64_t{1} << 31) - 1;
   return p.a_rows > 0 && p.a_rows * row_bytes <= kMax && p.nrows_w * row_bytes <= kMax;
 }
@@ -1020,13 +1027,18 @@ static bool wide_early_a_choice(const GemmParams& p) {
   return p.num_experts > 0 && p.numel >= 512LL * p.num_experts;
 }
 
+// Column tiles of a launch (a GEMM2's last one may hold half the columns).
+static int wide_col_tiles(bool gemm1, const GemmParams& p) {
+  const int cols = gemm1 ? WideRing::BNR / 2 : WideRing::BNR;
+  return static_cast<int>((p.n_out + cols - 1) / cols);
+}
+
 // A launch's normalised parameters (k split, tail split, whether it has a
 // plan) and the positions per XCD its whole tiles may take: the even split
 // needs total / 8; a cost-balanced plan may give an XCD up to a quarter more
 // (the plan falls back to the even split beyond that).
 static void wide_launch_shape(bool gemm1, const GemmParams& p, int row_blocks, GemmParams* q,
                               int64_t* cap) {
-  using C = WideRing;
   *q = p;
   q->row_blocks = row_blocks;
   if (gemm1 || q->ksplit < 1) q->ksplit = 1;
@@ -1034,21 +1046,20 @@ static void wide_launch_shape(bool gemm1, const GemmParams& p, int row_blocks, G
   if (q->tail_split) q->ksplit = 1;
   // the plan: few row blocks, whole tiles (see wide_plan_kernel)
   if (row_blocks > kPlanMaxRows || q->ksplit > 1 || plan_off()) q->plan = nullptr;
-  const int n_ct = static_cast<int>(gemm1 ? p.n_out / (C::BNR / 2) : p.n_out / C::BNR);
+  const int n_ct = wide_col_tiles(gemm1, p);
   const int64_t total = static_cast<int64_t>(row_blocks) * q->ksplit * n_ct;
   *cap = (total + 7) / 8;
   if (q->plan) *cap = *cap * 5 / 4 + 1;
 }
 
 void wide_plan_request(bool gemm1, const GemmParams& p, int row_blocks, WidePlanReq* req) {
-  using C = WideRing;
   GemmParams q;
   int64_t cap;
   wide_launch_shape(gemm1, p, row_blocks, &q, &cap);
   *req = WidePlanReq{};
   if (!q.plan) return;
   req->plan = q.plan;
-  req->n_ct = static_cast<int32_t>(gemm1 ? p.n_out / (C::BNR / 2) : p.n_out / C::BNR);
+  req->n_ct = wide_col_tiles(gemm1, p);
   req->cap = static_cast<int32_t>(cap);
   req->base = gemm1 ? kPlanBaseGemm1 : kPlanBaseGemm2;
 }
@@ -1068,15 +1079,14 @@ static int launch_wide_t(const GemmParams& p, int row_blocks, hipStream_t stream
   int64_t cap;
   wide_launch_shape(GEMM1, p, row_blocks, &q, &cap);
   set_topk_magic(&q);
-  const int n_ct_walk = static_cast<int>(GEMM1 ? p.n_out / (C::BNR / 2) : p.n_out / C::BNR);
+  const int n_ct = wide_col_tiles(GEMM1, p);
   const double rows_per_expert =
       p.num_experts > 0 ? static_cast<double>(p.numel) / p.num_experts : 0.0;
   if (q.group_n < 1)
-    q.group_n = wide_group_n_choice(GEMM1, n_ct_walk, rows_per_expert, q.plan != nullptr);
+    q.group_n = wide_group_n_choice(GEMM1, n_ct, rows_per_expert, q.plan != nullptr);
   // enough positions for the largest XCD walk the kernel can form from the
   // launched row blocks (it splits the live ones, known on the device), and
   // for the tail pieces of its last round
-  const int n_ct = static_cast<int>(GEMM1 ? p.n_out / (C::BNR / 2) : p.n_out / C::BNR);
   int64_t extra = 0;  // positions past an XCD's range (claims of others' tails)
   if (q.plan) {
     extra = GEMM1 ? 32 : 0;

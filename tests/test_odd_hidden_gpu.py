@@ -1,0 +1,63 @@
+"""Hidden sizes that are an odd multiple of 128 on the tiled schedules: GEMM2's
+256-column tiles end in a half tile there. Every tiled configuration against
+the oracle (the tolerances of test_fused_moe_gpu.py) and bit for bit against
+each other, the split tail and the k split on half tiles, and the
+allocation-free entry point where only the streaming workspace fits."""
+
+import pytest
+import torch
+
+from flaggems_sglang import _capi, testing
+from flaggems_sglang.ops import fused_moe as fm
+from oracle import moe_ref
+from test_fused_moe_gpu import _bias_inputs, _check, _routing_with_counts, _sample
+from test_zz_no_alloc import _no_alloc, _with_workspace
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("mode,K,N", [("bf16", 128, 256), ("bf16", 384, 128), ("bf16", 1152, 384),
+                                      ("fp8", 128, 256), ("fp8", 640, 384)])
+def test_odd_hidden_tiled_configs(gpu, mode, K, N):
+    rem = [1, 33, 128, 160, 161, 255, 64, 0]
+    counts = [256 * (e % 2) + r for e, r in enumerate(rem)]
+    w, ids = _routing_with_counts(counts, gpu, seed=N)
+    wts = testing.make_weights(K, N, len(counts), mode, 0.05, device=gpu, seed=K + N)
+    g = torch.Generator(device=gpu).manual_seed(K)
+    x = torch.randn(ids.shape[0], K, generator=g, device=gpu).to(torch.bfloat16)
+    ref = moe_ref.fused_moe(x, wts.w1, wts.w2, w, ids, mode=mode, w1_scale=wts.w1_scale,
+                            w2_scale=wts.w2_scale, return_mag=True)
+    outs = [fm.fused_moe(x, wts.w1, wts.w2, w, ids, _flags=_capi.flag_tile(cfg),
+                         **wts.kwargs(mode)) for cfg in range(_capi.TILED_CONFIGS)]
+    # (fp8: every token, as in test_block_remainders, so its bound of 8 ulps)
+    _check(outs[0].cpu(), ref, mode, f"odd hidden {K} {N} {mode}",
+           ulp_mag=8.0 if mode == "fp8" else None)
+    for cfg in range(1, _capi.TILED_CONFIGS):
+        assert torch.equal(outs[0], outs[cfg]), f"{mode} K={K} N={N}: tile 0 vs tile {cfg}"
+
+
+# (2100, 4224, ...): 1 to 8 rounds of tiles, the split tail; (700, 1408, ...):
+# a k split of 128-row tiles; the default schedule of each
+@pytest.mark.parametrize("shape", [(2100, 4224, 512, 8, 2), (700, 1408, 2048, 16, 1)])
+def test_odd_hidden_splits(gpu, shape):
+    M, K, N, E, topk = shape
+    x, w1, w2, b1, b2, w, ids = _bias_inputs(M, K, N, E, topk, gpu)
+    toks = _sample(M, 48)
+    res = fm.fused_moe(x, w1, w2, w, ids)
+    ref = moe_ref.fused_moe(x, w1, w2, w, ids, tokens=toks, return_mag=True)
+    _check(res.cpu()[toks], ref, "bf16", f"odd hidden {shape}")
+    res = fm.fused_moe_with_bias(x, w1, b1, w2, b2, w, ids, interleaved=False)
+    ref = moe_ref.fused_moe(x, w1, w2, w, ids, tokens=toks, return_mag=True,
+                            activation="swiglu", b1=b1, b2=b2)
+    _check(res.cpu()[toks], ref, "bf16", f"odd hidden bias {shape}")
+
+
+def test_odd_hidden_no_alloc_streams(gpu):
+    """The tiled schedule's split-tail workspace alone is the whole device
+    scratch; the streaming one fits, and the call is still served."""
+    M, K, N, E, topk = 2048, 4224, 256, 8, 2
+    wts = testing.make_weights(K, N, E, "bf16", 0.05, device=gpu, seed=K)
+    x, w, ids = testing.make_tokens(M, K, E, topk, device=gpu)
+    out = _no_alloc(x, wts.w1, wts.w2, w, ids)
+    ref = _with_workspace(x, wts.w1, wts.w2, w, ids, flags=_capi.FLAG_FORCE_DECODE)
+    assert torch.equal(out, ref)

@@ -99,16 +99,20 @@ __device__ __forceinline__ float gelu_mul(float g, float u) {
 // bf16(g * sigmoid(alpha * g) * (u + 1)), times the router weight when it
 // goes on the input (matmul_ogs scales its epilogue's output -- the fused
 // activation's result -- by the gammas).
+__device__ __forceinline__ float swiglu_mul(float g, float u, float alpha, float limit) {
+  if (limit > 0.f) {
+    g = fminf(g, limit);
+    u = fminf(fmaxf(u, -limit), limit);
+  }
+  const float sg = __builtin_amdgcn_rcpf(1.0f + __expf(-alpha * g));
+  return g * sg * (u + 1.0f);
+}
+
 __device__ __forceinline__ uint16_t gemm1_epilogue(float g, float u, bool scale,
                                                    float gamma, int act = kActSilu,
                                                    float alpha = 1.f, float limit = 0.f) {
   if (act == kActSwiglu) {
-    if (limit > 0.f) {
-      g = fminf(g, limit);
-      u = fminf(fmaxf(u, -limit), limit);
-    }
-    const float sg = __builtin_amdgcn_rcpf(1.0f + __expf(-alpha * g));
-    const float o = g * sg * (u + 1.0f);
+    const float o = swiglu_mul(g, u, alpha, limit);
     return f32_to_bf16_bits(scale ? o * gamma : o);
   }
   if (scale) {
@@ -121,25 +125,32 @@ __device__ __forceinline__ uint16_t gemm1_epilogue(float g, float u, bool scale,
 }
 
 
-// gemm1_epilogue's silu path for two adjacent outputs, word-packed: the same
-// roundings (g and u to bf16, silu(g) * u in fp32, bf16 out) with the
-// conversions done pairwise.
-template <bool SCALE>
-__device__ __forceinline__ uint32_t silu_mul_bf16x2(float g0, float g1, float u0, float u1,
-                                                    float gamma) {
-  if (SCALE) {
-    g0 *= gamma;
-    g1 *= gamma;
-    u0 *= gamma;
-    u1 *= gamma;
+// gemm1_epilogue for two adjacent outputs, word-packed, with the activation
+// and the router-weight scaling at compile time: the same roundings, the
+// conversions done pairwise (g and u already hold any bias).
+template <int ACT, bool SCALE>
+__device__ __forceinline__ uint32_t gemm1_epilogue_bf16x2(float g0, float g1, float u0, float u1,
+                                                          float gamma, float alpha = 1.f,
+                                                          float limit = 0.f) {
+  if constexpr (ACT == kActSwiglu) {
+    const float o0 = swiglu_mul(g0, u0, alpha, limit);
+    const float o1 = swiglu_mul(g1, u1, alpha, limit);
+    return SCALE ? cvt_pk_bf16(o0 * gamma, o1 * gamma) : cvt_pk_bf16(o0, o1);
+  } else {
+    if (SCALE) {
+      g0 *= gamma;
+      g1 *= gamma;
+      u0 *= gamma;
+      u1 *= gamma;
+    }
+    const uint32_t gp = cvt_pk_bf16(g0, g1);
+    const uint32_t up = cvt_pk_bf16(u0, u1);
+    auto act = [](float g, float u) { return ACT == kActGelu ? gelu_mul(g, u) : silu_mul(g, u); };
+    const float o0 = act(__builtin_bit_cast(float, gp << 16), __builtin_bit_cast(float, up << 16));
+    const float o1 = act(__builtin_bit_cast(float, gp & 0xffff0000u),
+                         __builtin_bit_cast(float, up & 0xffff0000u));
+    return cvt_pk_bf16(o0, o1);
   }
-  const uint32_t gp = cvt_pk_bf16(g0, g1);
-  const uint32_t up = cvt_pk_bf16(u0, u1);
-  const float o0 = silu_mul(__builtin_bit_cast(float, gp << 16),
-                            __builtin_bit_cast(float, up << 16));
-  const float o1 = silu_mul(__builtin_bit_cast(float, gp & 0xffff0000u),
-                            __builtin_bit_cast(float, up & 0xffff0000u));
-  return cvt_pk_bf16(o0, o1);
 }
 
 // ------------------------------------------------------------------ MFMA ---

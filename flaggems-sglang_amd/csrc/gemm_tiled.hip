@@ -699,10 +699,10 @@ __device__ __forceinline__ void tiled_tile(const GemmParams& p, const int rb_id,
                 const Acc& au = acc[i][jb + CB / 2];
                 const int v = 4 * g4;
                 uint2 v2;
-                v2.x = silu_mul_bf16x2<SCALE>(
+                v2.x = gemm1_epilogue_bf16x2<kActSilu, SCALE>(
                     value(ag, v, sa, sg[0]), value(ag, v + 1, sa, sg[1]),
                     value(au, v, sa, su[0]), value(au, v + 1, sa, su[1]), gamma);
-                v2.y = silu_mul_bf16x2<SCALE>(
+                v2.y = gemm1_epilogue_bf16x2<kActSilu, SCALE>(
                     value(ag, v + 2, sa, sg[2]), value(ag, v + 3, sa, sg[3]),
                     value(au, v + 2, sa, su[2]), value(au, v + 3, sa, su[3]), gamma);
                 *reinterpret_cast<uint2*>(slot_at(ch, r, jl * 4 + g4) + half * 8) = v2;

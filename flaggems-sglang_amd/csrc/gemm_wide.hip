@@ -252,7 +252,7 @@ __device__ __forceinline__ WideRange wide_range(const GemmParams& p, int total, 
   return w;
 }
 
-template <int DT, bool GEMM1, class C>
+template <int DT, bool GEMM1, class C, int ACT = kActSilu>
 __global__ __launch_bounds__(C::NW * 64, 1) void moe_gemm_wide_kernel(const GemmParams p) {
   using T = TiledType<DT>;
   using Frag = typename T::Frag;
@@ -651,8 +651,8 @@ __global__ __launch_bounds__(C::NW * 64, 1) void moe_gemm_wide_kernel(const Gemm
       // counts stores too, so a global load issued after one block's stores
       // would wait for them to complete. Table (floats): [0, 128) column
       // scales (GEMM1: 64 gate, 64 up), [128, 256) bias (GEMM2) or router
-      // weights (GEMM1), [256, 384) token slots, [384, 512) row scales;
-      // row (block i, r) at i * 32 + r.
+      // weights (GEMM1), [256, 384) token slots (GEMM2) or bias (GEMM1: 64
+      // gate, 64 up), [384, 512) row scales; row (block i, r) at i * 32 + r.
       // (in stage KT-2's slot of the two-slot ring)
       float* tab = reinterpret_cast<float*>(lds + R2 + ((KT - 2) % 2) * SLOT + wave * C::TAB_BYTES);
       int* tsid = reinterpret_cast<int*>(tab + 256);
@@ -667,7 +667,7 @@ __global__ __launch_bounds__(C::NW * 64, 1) void moe_gemm_wide_kernel(const Gemm
           const int sid = p.sorted_ids[row0 + rr];
           const bool ok = sid < p.numel;
           const int t = i * 32 + (lane & 31);
-          tsid[t] = sid;
+          if constexpr (!GEMM1) tsid[t] = sid;
           if constexpr (INT8)
             tab[384 + t] = p.a_scale[GEMM1 ? (ok ? div_topk(p, sid) : 0) : row0 + (ok ? rr : 0)];
           if (woi) tab[128 + t] = ok ? p.topk_w[sid] : 1.f;
@@ -678,10 +678,11 @@ __global__ __launch_bounds__(C::NW * 64, 1) void moe_gemm_wide_kernel(const Gemm
         else return 1.f;
       };
       if constexpr (GEMM1) {
-        // silu, no bias (the launch guarantees both): 64 output columns per
-        // wave, 128-byte staged rows (8 chunks). The router-weight scaling is
-        // a compile-time branch so the common case carries no per-element
-        // select.
+        // 64 output columns per wave, 128-byte staged rows (8 chunks). The
+        // activation and the router-weight scaling are compile-time branches
+        // so the common case carries no per-element select; the bias goes
+        // with swiglu and only with it (the launch guarantees it).
+        constexpr bool BIAS = ACT == kActSwiglu;
         constexpr int CH = WCOLS / 2 / 8;  // chunks per staged row
         uint16_t* out = static_cast<uint16_t*>(p.out);
         const int col_base = cur.ct * (BNR / 2) + wn * (WCOLS / 2);
@@ -690,7 +691,17 @@ __global__ __launch_bounds__(C::NW * 64, 1) void moe_gemm_wide_kernel(const Gemm
           tab[lane] = wsc[col_base + lane];
           tab[64 + lane] = wsc[p.n_out + col_base + lane];
         }
+        if constexpr (BIAS) {
+          const float* bias = p.bias + wbase + col_base;
+          tab[256 + lane] = bias[lane];
+          tab[320 + lane] = bias[p.n_out + lane];
+        }
         stage_sync();
+        auto cb4 = [&](int c) -> f32x4 {
+          if constexpr (BIAS) return *reinterpret_cast<const f32x4*>(tab + 256 + c);
+          else return f32x4{0.f, 0.f, 0.f, 0.f};
+        };
+        auto with_b = [](float x, float b) { return BIAS ? x + b : x; };
         auto csc4 = [&](int c) -> f32x4 {
           if constexpr (INT8) return *reinterpret_cast<const f32x4*>(tab + c);
           else return f32x4{1.f, 1.f, 1.f, 1.f};
@@ -708,16 +719,22 @@ __global__ __launch_bounds__(C::NW * 64, 1) void moe_gemm_wide_kernel(const Gemm
               for (int g4 = 0; g4 < 4; ++g4) {
                 const f32x4 swg = csc4(jb * 32 + csub + 8 * g4);
                 const f32x4 swu = csc4(64 + jb * 32 + csub + 8 * g4);
+                const f32x4 bg = cb4(jb * 32 + csub + 8 * g4);
+                const f32x4 bu = cb4(64 + jb * 32 + csub + 8 * g4);
                 const Acc& ag = acc[i][jb];
                 const Acc& au = acc[i][jb + CB / 2];
                 const int v = 4 * g4;
+                auto pair = [&](int t) -> uint32_t {
+                  return gemm1_epilogue_bf16x2<ACT, SCALE>(
+                      with_b(value(ag, v + t, sa, swg[t]), bg[t]),
+                      with_b(value(ag, v + t + 1, sa, swg[t + 1]), bg[t + 1]),
+                      with_b(value(au, v + t, sa, swu[t]), bu[t]),
+                      with_b(value(au, v + t + 1, sa, swu[t + 1]), bu[t + 1]), gamma, p.alpha,
+                      p.limit);
+                };
                 uint2 v2;
-                v2.x = silu_mul_bf16x2<SCALE>(
-                    value(ag, v, sa, swg[0]), value(ag, v + 1, sa, swg[1]),
-                    value(au, v, sa, swu[0]), value(au, v + 1, sa, swu[1]), gamma);
-                v2.y = silu_mul_bf16x2<SCALE>(
-                    value(ag, v + 2, sa, swg[2]), value(ag, v + 3, sa, swg[3]),
-                    value(au, v + 2, sa, swu[2]), value(au, v + 3, sa, swu[3]), gamma);
+                v2.x = pair(0);
+                v2.y = pair(2);
                 const int c = jb * 4 + g4;
                 *reinterpret_cast<uint2*>(stg + r * (CH * 16) + ((c ^ (r % CH)) * 16) + half * 8) = v2;
               }
@@ -962,15 +979,18 @@ int64_t wide_tail_part_bytes() {
 }
 
 // Whether the 4-wave kernel covers a launch: bf16 / int8, GEMM1 with
-// the silu activation and no bias (gelu and the swiglu bias variant keep the
-// 8-wave kernel), k split into >= 2 stages per split, output tiles that
+// silu or gelu and no bias or the bias variant's swiglu (the last two also
+// ran the 8-wave kernel, whose epilogue stores them 8 bytes a lane, 32 rows
+// per instruction; here, same box: gelu on Qwen3 M=2048 450 -> 346 us, Mixtral
+// M=4096 2.70 -> 2.60 ms; swiglu with bias, hidden 3072, intermediate 2048, 64
+// experts, top-8, 2048 tokens 996 -> 812 us), k split into >= 2 stages per split, output tiles that
 // divide n_out, and operands whose byte offsets fit the 32-bit buffer
 // addressing.
 bool wide_supported(int dt, bool gemm1, const GemmParams& p) {
   using C = WideRing;
   if (dt != kDtBf16 && dt != kDtInt8) return false;
   if (p.eid_shift != 0) return false;  // row blocks are whole alignment blocks
-  if (gemm1 && (p.act != kActSilu || p.bias != nullptr)) return false;
+  if (gemm1 && (p.act == kActSwiglu) != (p.bias != nullptr)) return false;
   const int64_t esz = dt == kDtBf16 ? 2 : 1;
   const int64_t row_bytes = p.kdim * esz;
   if (row_bytes % C::SK != 0) return false;
@@ -1064,9 +1084,9 @@ void wide_plan_request(bool gemm1, const GemmParams& p, int row_blocks, WidePlan
   req->base = gemm1 ? kPlanBaseGemm1 : kPlanBaseGemm2;
 }
 
-template <int DT, bool GEMM1, class C>
+template <int DT, bool GEMM1, class C, int ACT = kActSilu>
 static int launch_wide_t(const GemmParams& p, int row_blocks, hipStream_t stream) {
-  auto kern = moe_gemm_wide_kernel<DT, GEMM1, C>;
+  auto kern = moe_gemm_wide_kernel<DT, GEMM1, C, ACT>;
   static std::once_flag once;
   static hipError_t attr = hipSuccess;
   std::call_once(once, [&] {
@@ -1109,20 +1129,31 @@ static int launch_wide_t(const GemmParams& p, int row_blocks, hipStream_t stream
   return check_launch("moe_wide_tail_fixup_kernel");
 }
 
+template <int DT>
+static int launch_wide_gemm1(const GemmParams& p, int row_blocks, hipStream_t stream) {
+  switch (p.act) {
+    case kActGelu: return launch_wide_t<DT, true, WideRing, kActGelu>(p, row_blocks, stream);
+    case kActSwiglu: return launch_wide_t<DT, true, WideRing, kActSwiglu>(p, row_blocks, stream);
+    default: return launch_wide_t<DT, true, WideRing>(p, row_blocks, stream);
+  }
+}
+
+template <int DT>
+static int launch_wide_gemm2(const GemmParams& p, int row_blocks, hipStream_t stream) {
+  return wide_early_a_choice(p) ? launch_wide_t<DT, false, WideRingA>(p, row_blocks, stream)
+                                : launch_wide_t<DT, false, WideRing>(p, row_blocks, stream);
+}
+
 int launch_gemm_wide(int dt, bool gemm1, const GemmParams& p, int row_blocks,
                      hipStream_t stream) {
   if (!wide_supported(dt, gemm1, p))
     return fail(FGS_EINVAL, "wide GEMM: launch not covered by the 4-wave kernel");
   if (row_blocks <= 0) return FGS_OK;
-  const bool early_a = !gemm1 && wide_early_a_choice(p);
-  if (dt == kDtBf16) {
-    if (gemm1) return launch_wide_t<kDtBf16, true, WideRing>(p, row_blocks, stream);
-    return early_a ? launch_wide_t<kDtBf16, false, WideRingA>(p, row_blocks, stream)
-                   : launch_wide_t<kDtBf16, false, WideRing>(p, row_blocks, stream);
-  }
-  if (gemm1) return launch_wide_t<kDtInt8, true, WideRing>(p, row_blocks, stream);
-  return early_a ? launch_wide_t<kDtInt8, false, WideRingA>(p, row_blocks, stream)
-                 : launch_wide_t<kDtInt8, false, WideRing>(p, row_blocks, stream);
+  if (dt == kDtBf16)
+    return gemm1 ? launch_wide_gemm1<kDtBf16>(p, row_blocks, stream)
+                 : launch_wide_gemm2<kDtBf16>(p, row_blocks, stream);
+  return gemm1 ? launch_wide_gemm1<kDtInt8>(p, row_blocks, stream)
+               : launch_wide_gemm2<kDtInt8>(p, row_blocks, stream);
 }
 
 }  // namespace fgs

@@ -1,8 +1,10 @@
-"""Hidden sizes that are an odd multiple of 128 on the tiled schedules: GEMM2's
-256-column tiles end in a half tile there. Every tiled configuration against
-the oracle (the tolerances of test_fused_moe_gpu.py) and bit for bit against
-each other, the split tail and the k split on half tiles, and the
-allocation-free entry point where only the streaming workspace fits."""
+"""Shapes and epilogues the tiled schedules took over from slower ones.
+
+Hidden sizes that are an odd multiple of 128: GEMM2's 256-column tiles end in
+a half tile there. Every tiled configuration against the oracle (the
+tolerances of test_fused_moe_gpu.py) and bit for bit against each other, the
+split tail and the k split on half tiles, and the allocation-free entry point
+where only the streaming workspace fits. gelu and swiglu on the 4-wave kernel."""
 
 import pytest
 import torch
@@ -61,3 +63,40 @@ def test_odd_hidden_no_alloc_streams(gpu):
     out = _no_alloc(x, wts.w1, wts.w2, w, ids)
     ref = _with_workspace(x, wts.w1, wts.w2, w, ids, flags=_capi.FLAG_FORCE_DECODE)
     assert torch.equal(out, ref)
+
+
+@pytest.mark.parametrize("on_input", [False, True], ids=["gammas_out", "gammas_in"])
+@pytest.mark.parametrize("mode", ["bf16", "int8"])
+@pytest.mark.parametrize("act", ["gelu", "swiglu"])
+def test_wide_activations(gpu, act, mode, on_input):
+    """gelu and the bias variant's swiglu in the 4-wave kernel's epilogue
+    (256-row blocks, every partial block) against the oracle and the 8-wave
+    kernels' epilogues, which round at the same points."""
+    K, N = 512, 256
+    rem = [1, 33, 128, 160, 161, 255, 64, 0]
+    counts = [256 * (e % 2) + r for e, r in enumerate(rem)]
+    w, ids = _routing_with_counts(counts, gpu, seed=N)
+    M, E = ids.shape[0], len(counts)
+    wts = testing.make_weights(K, N, E, mode, 0.05, device=gpu, seed=K + N)
+    g = torch.Generator(device=gpu).manual_seed(K)
+    x = torch.randn(M, K, generator=g, device=gpu).to(torch.bfloat16)
+    b1 = torch.randn(E, 2 * N, generator=g, device=gpu) * 0.5
+    b2 = torch.randn(E, K, generator=g, device=gpu) * 0.5
+
+    def run(cfg):
+        kw = dict(apply_router_weight_on_input=on_input, _flags=_capi.flag_tile(cfg),
+                  **wts.kwargs(mode))
+        if act == "gelu":
+            return fm.fused_moe(x, wts.w1, wts.w2, w, ids, activation="gelu", **kw)
+        return fm.fused_moe_with_bias(x, wts.w1, b1, wts.w2, b2, w, ids, gemm1_alpha=1.702,
+                                      gemm1_clamp_limit=7.0, interleaved=False, **kw)
+
+    kw = dict(mode=mode, w1_scale=wts.w1_scale, w2_scale=wts.w2_scale, activation=act,
+              apply_router_weight_on_input=on_input, return_mag=True)
+    if act == "swiglu":
+        kw.update(b1=b1, b2=b2, alpha=1.702, limit=7.0)
+    ref = moe_ref.fused_moe(x, wts.w1, wts.w2, w, ids, **kw)
+    out = run(0)
+    _check(out.cpu(), ref, mode, f"wide {act} {mode} {on_input}")
+    for cfg in (1, 3):
+        assert torch.equal(out, run(cfg)), f"{act} {mode}: tile 0 vs tile {cfg}"

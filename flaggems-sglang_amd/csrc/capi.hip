@@ -63,6 +63,8 @@ struct Plan {
   bool tiled;      // LDS-tiled MFMA kernels (prefill) instead of streaming
   int tile_cfg;    // tiled kernel configuration
   int tile_cfg2;   // GEMM2's configuration (rows per block <= block_m)
+  int shape1, shape2;  // tile shape of GEMM1 / GEMM2 (kTileByConfig, ...)
+  int eid_shift1;  // log2(block_m / GEMM1 block rows)
   int eid_shift2;  // log2(block_m / GEMM2 block rows)
   int ksplit2;     // GEMM2 k splits (tiled only; > 1 -> fp32 partials)
   bool tail2;      // GEMM2 on the 4-wave kernel with its last round's tiles
@@ -82,21 +84,52 @@ struct Plan {
       total;
 };
 
-// k splits for the tiled GEMM2: its grid (row blocks x hidden/256 column
-// tiles) is often a few waves of 256 workgroups, and a partial last wave
-// idles most CUs for a whole tile. Pick the smallest split (<= 4, keeping
-// >= 8 LDS stages of 128 bytes of k per split) whose expected grid fills
-// >= 90 % of its last wave, else the best one. Row blocks are estimated for
-// balanced routing: numel / B plus half a padded block per touched expert.
 constexpr int kNumCUs = 256;  // MI355X
 
-static int pick_ksplit(int64_t numel, int e, int bm, int64_t hidden,
-                       int64_t k_bytes, bool one_block_per_expert = false) {
-  const double blocks = one_block_per_expert
-                            ? static_cast<double>(std::min<int64_t>(e, numel))
-                            : static_cast<double>(numel) / bm +
-                                  0.5 * static_cast<double>(std::min<int64_t>(e, numel));
-  const double wgs = blocks * static_cast<double>((hidden + 255) / 256);
+// Row blocks of bm rows the alignment is expected to make: an expert's slots
+// are about normal around numel / e (each token picks an expert with
+// probability topk / e), and it holds a j-th block when it has more than
+// (j - 1) * bm slots.
+static double expected_blocks(int64_t m, int topk, int e, int bm) {
+  const double mean = static_cast<double>(m) * topk / e;
+  const double sd = std::sqrt(std::max(1e-3, mean * (1.0 - static_cast<double>(topk) / e)));
+  double per_expert = 1.0 - std::exp(-mean);
+  for (double at = bm; at <= mean + 6 * sd; at += bm)
+    per_expert += 0.5 * std::erfc((at + 0.5 - mean) / (sd * std::sqrt(2.0)));
+  return std::min(per_expert * e, static_cast<double>(m) * topk);
+}
+
+// k splits of the tiled GEMM2, for a grid that leaves CUs without a tile:
+// a split saves (1 - 1/s) of a tile's k stages (~0.9 us each) and costs its
+// fp32 partials (8 bytes written and read per output and split, against 4
+// for bf16 rows, at ~4 TB/s) and ~3 us of the slower sum; at least 8 stages
+// stay per split. Splitting a grid that covers the CUs to fill its last
+// round costs more than it saves (measured at 256 rows per expert, one box:
+// fp8 hidden 1280, intermediate 3072, 64 experts GEMM2 and sum 260 us with
+// the split that filled the last round, 147 without; Mixtral's long rows at
+// 32 tokens per expert 246 us unsplit, 174 in two).
+static int pick_ksplit(double tiles, int64_t stages, int64_t numel, int64_t hidden) {
+  int best = 1;
+  double best_gain = 0.0;
+  for (int s = 2; s <= 4; ++s) {
+    if (stages < 8 * s || tiles * s > 1.1 * kNumCUs) break;
+    const double gain = 0.9 * static_cast<double>(stages) * (1.0 - 1.0 / s) - 3.0 -
+                        static_cast<double>(numel) * static_cast<double>(hidden) * (8 * s - 4) / 4e6;
+    if (gain > best_gain) {
+      best_gain = gain;
+      best = s;
+    }
+  }
+  return best;
+}
+
+// The k split the allocation-free entry point's scratch is sized for
+// (scratch_rule): the smallest (<= 4, keeping >= 8 stages of 128 bytes of k)
+// whose expected grid fills >= 90 % of its last round, else the best one.
+static int scratch_ksplit(int64_t numel, int e, int bm, int64_t hidden, int64_t k_bytes) {
+  const double blocks = static_cast<double>(numel) / bm +
+                        0.5 * static_cast<double>(std::min<int64_t>(e, numel));
+  const double wgs = blocks * static_cast<double>(hidden / 256);
   int best = 1;
   double best_eff = 0.0;
   for (int s = 1; s <= 4; ++s) {
@@ -180,76 +213,168 @@ static int pick_kw(int64_t kdim, int step, int cap, int min_steps) {
   return kw;
 }
 
-static int make_plan(int64_t m, int64_t hidden, int64_t inter, int e, int topk,
-                     int qmode, int flags, Plan* pl) {
+// Rows per expert up to which a call streams, by GEMM1's 128-column tiles
+// over the touched experts (`k_bytes`: GEMM2's k row). The tiled kernels'
+// pipeline pays off earlier the more tiles share its fill, and the small
+// grids have the 128x128 tiles. Layer time, streaming / tiled, over weights
+// rotated through more memory than the caches (rows per expert: ratio):
+// bf16 48 tiles 10: 1.01, 12: 1.04; 64 8: 0.96, 10: 1.05; 112 10: 0.99, 12:
+// 1.06; 128 10: 0.93, 12: 1.00; 768 (1.5 KiB k rows) 12: 0.93, 14: 1.10; 736
+// 8: 0.97, 10: 1.03; 896 8: 0.94, 10: 0.98, 12: 1.09; 1280 6: 0.97, 8:
+// 1.01; 1536 6: 0.93, 8: 0.99; 1920 6: 0.98, 8: 1.02; 2944 6: 1.00, 8:
+// 1.04. int8 48 tiles 12: 0.98, 14: 1.04; 112 12: 0.96, 14: 1.09; 128 12:
+// 0.95, 14: 1.06; 768 4: 1.00, 6: 1.03; 704 6: 0.98, 8: 0.99, 10: 1.03; 896
+// 6: 0.99, 8: 1.02; 1280 4: 1.00, 6: 1.07; 1536 4: 1.03; 1920 6: 1.00, 8:
+// 1.03; 2816 4: 1.07. fp8 48 tiles 8: 1.00, 14: 1.08; 112 4: 0.97, 8: 1.02;
+// 128 8: 0.95, 10: 1.02; 736 and more 4: 1.03 to 1.15.
+static double stream_rows(int dt, double tiles, int64_t k_bytes) {
+  if (dt == kDtFp8) return tiles <= 160 ? 7 : 3;
+  if (dt == kDtInt8) return tiles <= 160 ? 12.5 : tiles <= 1000 ? 6 : tiles <= 2000 ? 4.5 : 3;
+  return tiles <= 160 ? 10 : tiles <= 1000 ? (k_bytes < 2048 ? 12.5 : 9) : tiles <= 2000 ? 7 : 5.5;
+}
+
+// The schedule of a call with many rows: streaming or tiled, the tile
+// configuration and shape of each GEMM, GEMM2's split.
+//
+// Measured per GEMM with every schedule forced, cold caches, on one box: 11
+// layers of 8 to 160 experts (hidden 1024..7168, intermediate 512..14336),
+// 2 to 512 rows per expert, the three element types.
+static void call_rule(int64_t m, int64_t hidden, int64_t inter, int e, int topk, int flags,
+                      Plan* pl) {
+  Plan& p = *pl;
   const int64_t numel = m * topk;
-  Plan p{};
-  p.dt = qmode == FGS_QMODE_FP8_BLOCK ? kDtFp8
-         : qmode == FGS_QMODE_INT8_CHANNEL ? kDtInt8 : kDtBf16;
-  const double rows_per_expert = static_cast<double>(numel) / e;
-  p.mt = rows_per_expert <= 16 ? 1 : rows_per_expert <= 32 ? 2 : 4;
-  p.block_m = 16 * p.mt;
-  // LDS-tiled kernels (deep DMA pipeline) or the streaming kernels (weights
-  // straight into registers), by the rows per expert at which the tiled
-  // kernels' pipeline fill pays off, measured per element type and
-  // contraction length (kmin: the shorter of the two GEMMs' k rows in
-  // bytes), both schedules forced on the same box:
-  // * fp8 from 3 rows per expert (DeepSeek: streaming -6 % at 2 rows,
-  //   level at 3, tiled -1 % at 4);
-  // * a short k row (< 2 KiB, Qwen3) from 16 (streaming -10 % at 12 rows,
-  //   +4 % with skewed routing; tiled -9 % at 16);
-  // * a long one (>= 8 KiB, Mixtral) from 12 (streaming -9 % at 8 rows,
-  //   tiled -6 % at 12);
-  // * else (Qwen2 int8) from 8 (streaming -11 % at 6 rows, level at 8,
-  //   tiled -8 % at 12).
+  const int64_t esz = p.dt == kDtBf16 ? 2 : 1;
+  const double rows = static_cast<double>(numel) / e;
+  const int forced_cfg = ((flags & FGS_FLAG_TILE_MASK) >> 12) - 1;
+  // Streaming row blocks: 16 rows up to 12 rows per expert (more would give
+  // a share of the experts a second block, which streams their weights
+  // again), 32 up to 28 (bf16 hidden 3584, intermediate 2560, 64 experts, 16
+  // rows: GEMM1 614 us in blocks of 16, 528 of 32), else 64.
+  p.mt = rows <= 12 ? 1 : rows <= 28 ? 2 : 4;
+  // Tiled kernels (deep DMA pipeline) or streaming ones (weights straight
+  // into registers), by rows per expert: see stream_rows.
+  const double tiles1 = e * (1.0 - std::exp(-rows)) * static_cast<double>(inter / 128);
+  const double stream_to = stream_rows(p.dt, tiles1, inter * esz);
   // One token always streams (its direct-row schedule). Every accepted shape
   // can run tiled: a hidden size that is an odd multiple of 128 ends GEMM2 in
   // a half tile. (Streaming reads an expert's weights once per block of at
   // most 64 rows: hidden 2944, intermediate 2944, 32 experts, top-4, 4096
   // tokens with bias 7.12 ms streaming, 1.05 ms tiled.)
-  const int64_t esz = p.dt == kDtBf16 ? 2 : 1;
-  const int forced_cfg = ((flags & FGS_FLAG_TILE_MASK) >> 12) - 1;
-  const int64_t kmin = std::min(hidden, inter) * esz;
-  double tiled_from = 8.0;
-  if (p.dt == kDtFp8) tiled_from = 3.0;
-  else if (kmin < 2048) tiled_from = 16.0;
-  else if (kmin >= 8192) tiled_from = 12.0;
-  const bool many_rows = m >= 2 && rows_per_expert >= tiled_from;
   p.tiled = !(flags & FGS_FLAG_FORCE_DECODE) &&
-            ((flags & FGS_FLAG_FORCE_PREFILL) || forced_cfg >= 0 || many_rows);
-  p.ksplit2 = 1;
-  if (p.tiled) {
-    p.tile_cfg = forced_cfg >= 0 ? forced_cfg : tiled_config_for(p.dt, rows_per_expert, e);
-    p.block_m = tiled_block_m(p.tile_cfg);
-    // fp8 GEMM2 runs its 128-row kernel on 256-row blocks (as two halves,
-    // the all-pad ones skipped): the 256-row fp8 tile spans only 128 weight
-    // rows, so GEMM2 would re-read each activation tile for twice as many
-    // column tiles
-    p.tile_cfg2 = p.tile_cfg;
-    p.eid_shift2 = 0;
-    if (p.dt == kDtFp8 && p.tile_cfg == 0 && forced_cfg < 0) {
-      p.tile_cfg2 = 1;
-      p.eid_shift2 = 1;
+            ((flags & FGS_FLAG_FORCE_PREFILL) || forced_cfg >= 0 ||
+             (m >= 2 && rows > stream_to));
+  if (!p.tiled) return;
+  const double blocks128 = expected_blocks(m, topk, e, 128);
+  const double blocks256 = expected_blocks(m, topk, e, 256);
+  const int64_t ct1 = inter / 128, ct2 = (hidden + 255) / 256;
+  const int64_t stages2 = inter * esz / 128;
+  if (forced_cfg >= 0) {
+    p.tile_cfg = forced_cfg;
+  } else {
+    p.tile_cfg = tiled_config_for(p.dt, rows, e, blocks256 * ct1, blocks128 * ct1);
+    // Grids of under a round of wide tiles: 128x128 tiles with a 5-slot ring
+    // (an expert's rows in 128-row blocks), one round of them. GEMM1, us
+    // wide / deep: bf16 hidden 4096, intermediate 1792, 8 experts 95 / 87 at
+    // 16 rows, 101 / 92 at 90; hidden 2048, intermediate 768 36 / 26, 43 /
+    // 32, and 56 / 33 at 180; 256 such tiles and more are slower (1024, 512,
+    // 16 experts, 180 rows: 25 wide, 30).
+    const double deep_limit = 0.875 * kNumCUs;
+    if (!tile_forced()) {
+      if (blocks128 * (inter / 64) <= deep_limit) {
+        p.tile_cfg = 1;
+        p.shape1 = kTileDeep;
+      }
+      if (p.tile_cfg == 1 && blocks128 * (hidden / 128) <= deep_limit) p.shape2 = kTileDeep;
+      // fp8 GEMM1 of many experts on 256-row blocks: 128x128 tiles, two
+      // workgroups per CU, on the blocks' halves, so one tile's prologue and
+      // epilogue run under the other's k loop (256 rows: intermediate 5888,
+      // 64 experts, hidden 1536 567 -> 528 us; 3072, hidden 1280 298 ->
+      // 272) -- but not where most experts' rows overflow a half by a few,
+      // which the 160-row ring takes in one tile (hidden 5120, intermediate
+      // 1536, 160 experts, 128 rows: 785 us there, 825 so).
+      if (p.dt == kDtFp8 && p.tile_cfg == 0 && e >= 32 && rows > 200) {
+        p.shape1 = kTileDual;
+        p.eid_shift1 = 1;
+      }
     }
-    // (the 160-row configuration, when forced, runs below 160 rows per
-    // expert: about one block per touched expert)
-    p.ksplit2 = pick_ksplit(numel, e, tiled_block_m(p.tile_cfg2), hidden, inter * esz,
-                            p.tile_cfg2 == 4 && rows_per_expert < 160);
-    // a forced split still keeps >= 8 LDS stages of k per split
-    if (forced_ksplit() > 0 && inter * esz / 128 >= 8 * forced_ksplit())
-      p.ksplit2 = forced_ksplit();
-    // GEMM2 of 256-row blocks (bf16 / int8) over 1 to 8 rounds of the CUs:
-    // the 4-wave kernel, whole tiles except the last round's, which are
-    // split over k (instead of splitting every tile: fp32 partials of a few
-    // tiles, not of all). Measured: the 4-wave kernel runs a 256 x 256 x 64
-    // stage in ~1.78 us against the 8-wave kernel's ~2.1 us on the dense
-    // Mixtral GEMM2, but left alone its tiles fill 2.25 rounds.
-    const int64_t rows_est = numel / 256 + std::min<int64_t>(e, numel);
-    const int64_t tiles_est = rows_est * ((hidden + 255) / 256);
-    p.tail2 = tail_choice() && p.tile_cfg2 == 0 && p.dt != kDtFp8 && forced_ksplit() == 0 &&
-              tiles_est >= kNumCUs && tiles_est <= 8 * kNumCUs;
-    if (p.tail2) p.ksplit2 = 1;
   }
+  // fp8 GEMM2 on 256-row blocks runs its 128-row kernel on their halves (the
+  // all-pad ones skipped): the 256-row fp8 tile spans only 128 weight rows,
+  // so it reads each activation tile for twice as many column tiles. At 128
+  // rows per expert its 160-row ring still wins on long k rows, where the
+  // second halves of a few rows would stream the weights again (layer, halves
+  // / 256-row: intermediate 5888 604 / 560 us, 2560 559 / 526, 14336 400 /
+  // 389; 2048 3032 / 3067, 768 253 / 267).
+  p.tile_cfg2 = p.tile_cfg;
+  if (p.dt == kDtFp8 && p.tile_cfg == 0 && forced_cfg < 0 && !(rows <= 200 && inter >= 2560)) {
+    p.tile_cfg2 = 1;
+    p.eid_shift2 = 1;
+  }
+  const int bm2 = tiled_block_m(p.tile_cfg2);
+  const double tiles2 = p.shape2 == kTileDeep ? blocks128 * static_cast<double>(hidden / 128)
+                        : expected_blocks(m, topk, e, bm2) *
+                              (p.dt == kDtFp8 && p.tile_cfg2 == 0
+                                   ? static_cast<double>(hidden / 128) : ct2);
+  p.ksplit2 = pick_ksplit(tiles2, stages2, numel, hidden);
+  // a forced split still keeps >= 8 LDS stages of k per split
+  if (forced_ksplit() > 0 && stages2 >= 8 * forced_ksplit()) p.ksplit2 = forced_ksplit();
+  // GEMM2 of 256-row blocks (bf16 / int8) over 1 to 8 rounds of the CUs:
+  // the 4-wave kernel, whole tiles except the last round's, which are split
+  // over k (fp32 partials of a few tiles, not of all; Mixtral at 128 rows
+  // per expert 185 us, 273 with whole tiles). From 40 stages of k: below,
+  // the partials and the fixup launch cost more than the shorter last round
+  // saves (28 stages, 8 experts, hidden 4096, 180 rows: 77 us split, 57
+  // whole; 22 stages int8, hidden 3072, 32 experts, 128 rows: 110 and 95; 12
+  // stages, hidden 2048, 128 experts, 256 rows: 216 and 195; 40..48 stages
+  // within 10 % either way; 92 stages 1..8 % faster split).
+  const int64_t rows_est = numel / 256 + std::min<int64_t>(e, numel);
+  const int64_t tiles_est = rows_est * ct2;
+  p.tail2 = tail_choice() && p.tile_cfg2 == 0 && p.dt != kDtFp8 && forced_ksplit() == 0 &&
+            stages2 >= 40 && tiles_est >= kNumCUs && tiles_est <= 8 * kNumCUs;
+  if (p.tail2) p.ksplit2 = 1;
+}
+
+// What the allocation-free entry point accepts: problems whose workspace
+// under this rule fits its fixed scratch. It serves them with the call's own
+// schedule where that fits as well, else with this one (smaller row blocks
+// and no split tail on some shapes), so the set does not move with call_rule.
+static void scratch_rule(int64_t m, int64_t hidden, int64_t inter, int e, int topk, int flags,
+                         Plan* pl) {
+  Plan& p = *pl;
+  const int64_t numel = m * topk;
+  const double rows = static_cast<double>(numel) / e;
+  const int forced_cfg = ((flags & FGS_FLAG_TILE_MASK) >> 12) - 1;
+  p.mt = rows <= 16 ? 1 : rows <= 32 ? 2 : 4;
+  const int64_t k_bytes = inter * 2;
+  const int64_t kmin = std::min(hidden * 2, k_bytes);
+  const double tiled_from = kmin < 2048 ? 16.0 : kmin >= 8192 ? 12.0 : 8.0;
+  p.tiled = hidden % 256 == 0 && !(flags & FGS_FLAG_FORCE_DECODE) &&
+            ((flags & FGS_FLAG_FORCE_PREFILL) || forced_cfg >= 0 ||
+             (m >= 2 && rows >= tiled_from));
+  if (!p.tiled) return;
+  const bool many = e >= 32;
+  p.tile_cfg = forced_cfg >= 0 ? forced_cfg
+               : rows >= 96 || (many && rows >= 48) ? 0
+               : rows >= 24 || (many && rows >= 8) ? 1 : 3;
+  p.tile_cfg2 = p.tile_cfg;
+  p.ksplit2 = scratch_ksplit(numel, e, tiled_block_m(p.tile_cfg), hidden, k_bytes);
+  const int64_t tiles_est = (numel / 256 + std::min<int64_t>(e, numel)) * (hidden / 256);
+  p.tail2 = p.tile_cfg == 0 && tiles_est >= kNumCUs && tiles_est <= 8 * kNumCUs;
+  if (p.tail2) p.ksplit2 = 1;
+}
+
+// `scratch`: the plan of scratch_rule (bf16) instead of the call's own.
+static int make_plan(int64_t m, int64_t hidden, int64_t inter, int e, int topk,
+                     int qmode, int flags, Plan* pl, bool scratch = false) {
+  const int64_t numel = m * topk;
+  Plan p{};
+  p.dt = qmode == FGS_QMODE_FP8_BLOCK ? kDtFp8
+         : qmode == FGS_QMODE_INT8_CHANNEL ? kDtInt8 : kDtBf16;
+  const int64_t esz = p.dt == kDtBf16 ? 2 : 1;
+  p.ksplit2 = 1;
+  if (scratch) scratch_rule(m, hidden, inter, e, topk, flags, &p);
+  else call_rule(m, hidden, inter, e, topk, flags, &p);
+  p.block_m = p.tiled ? tiled_block_m(p.tile_cfg) : 16 * p.mt;
   const int step = stream_step_k(p.dt);
   // GEMM1 on up to 4 waves; GEMM2 on as many as leave each wave 5 steps,
   // at least 2. Measured (same box, 3 x 20 flushed calls, twice): GEMM2 on
@@ -485,11 +610,13 @@ struct FusedArgs {
   const float* gate_scal = nullptr;
   const int32_t* gather_src = nullptr;
   const int32_t* expt_hist = nullptr;
+  // the schedule of scratch_rule (the allocation-free entry point)
+  bool scratch_plan = false;
 };
 
 static int run_fused(const FusedArgs& a) {
   int rc = validate(a.m, a.hidden, a.inter, a.e, a.topk, a.qmode, a.flags,
-                    a.ws_bytes, true);
+                    a.ws_bytes, !a.scratch_plan);
   if (rc) return rc;
   if (a.m == 0) return FGS_OK;  // nothing to read or write
   const bool routed = a.gather_src != nullptr;
@@ -505,7 +632,7 @@ static int run_fused(const FusedArgs& a) {
     return fail(FGS_EINVAL, "tensors must be 16-byte aligned (workspace 256)");
 
   Plan p;
-  make_plan(a.m, a.hidden, a.inter, a.e, a.topk, a.qmode, a.flags, &p);
+  make_plan(a.m, a.hidden, a.inter, a.e, a.topk, a.qmode, a.flags, &p, a.scratch_plan);
   uint8_t* ws = static_cast<uint8_t*>(a.ws);
   int32_t* sorted = reinterpret_cast<int32_t*>(ws + p.o_sorted);
   int32_t* eids = reinterpret_cast<int32_t*>(ws + p.o_eids);
@@ -610,7 +737,10 @@ static int run_fused(const FusedArgs& a) {
   g2.a_src = p.qfold ? a2 : nullptr;
   g2.a_scale_kstride = p.tiled && p.dt == kDtFp8 ? p.max_padded : 0;
   g2.plan = p.o_plan2 >= 0 ? reinterpret_cast<int32_t*>(ws + p.o_plan2) : nullptr;
-  const int rows1 = static_cast<int>(p.n_launch);
+  const int rows1 = static_cast<int>(p.n_launch << p.eid_shift1);
+  g1.eid_shift = p.tiled ? p.eid_shift1 : 0;
+  g1.shape = p.shape1;
+  g2.shape = p.shape2;
   const int rows2 = static_cast<int>(p.n_launch << p.eid_shift2);
 
   if (routed && !p.direct) {
@@ -929,6 +1059,9 @@ int32_t fgs_moe_schedule(int64_t m, int64_t hidden, int64_t inter, int32_t num_e
     s = "stream mt=" + std::to_string(p.mt);
   } else {
     s = "tiled cfg=" + std::to_string(p.tile_cfg) + " cfg2=" + std::to_string(p.tile_cfg2);
+    const char* shapes[] = {"", " deep", " dual"};
+    if (p.shape1) s += std::string(shapes[p.shape1]) + "1";
+    if (p.shape2) s += std::string(shapes[p.shape2]) + "2";
     if (p.ksplit2 > 1) s += " ksplit2=" + std::to_string(p.ksplit2);
     if (p.tail2) s += " tail2";
   }
@@ -1001,13 +1134,7 @@ int32_t fgs_moe_fused_bf16_noalloc(const void* x, const void* w13, const void* w
   int rc = validate(m, hidden, inter, num_experts, topk, FGS_QMODE_BF16, flags, 0, false);
   if (rc) return rc;
   Plan p;
-  make_plan(m, hidden, inter, num_experts, topk, FGS_QMODE_BF16, flags, &p);
-  // hidden sizes of an odd multiple of 128 keep the streaming schedule where
-  // only its smaller workspace (row blocks of at most 64, no split tail) fits
-  if (p.total > FGS_NOALLOC_SCRATCH_BYTES && p.tiled && hidden % 256 != 0) {
-    flags = (flags & ~(FGS_FLAG_FORCE_PREFILL | FGS_FLAG_TILE_MASK)) | FGS_FLAG_FORCE_DECODE;
-    make_plan(m, hidden, inter, num_experts, topk, FGS_QMODE_BF16, flags, &p);
-  }
+  make_plan(m, hidden, inter, num_experts, topk, FGS_QMODE_BF16, flags, &p, true);
   if (p.total > FGS_NOALLOC_SCRATCH_BYTES)
     return fail(FGS_EUNSUPPORTED,
                 "fgs_moe_fused_bf16_noalloc: this problem needs " + std::to_string(p.total) +
@@ -1034,6 +1161,9 @@ int32_t fgs_moe_fused_bf16_noalloc(const void* x, const void* w13, const void* w
               inter,          num_experts,  topk,     flags,  ws,
               FGS_NOALLOC_SCRATCH_BYTES, out, as_stream(stream)};
   a.no_profile = true;
+  Plan own;
+  make_plan(m, hidden, inter, num_experts, topk, FGS_QMODE_BF16, flags, &own);
+  a.scratch_plan = own.total > FGS_NOALLOC_SCRATCH_BYTES;
   return run_fused(a);
 }
 

@@ -16,6 +16,10 @@ enum : int { kDtBf16 = 0, kDtFp8 = 1, kDtInt8 = 2 };
 //          w = w2 [E, n_out, kdim], out = per-slot y bf16 [numel, n_out].
 constexpr int kQaMaxSlots = 64;  // on-the-fly quantisation: slots per call
 
+// Tile shape of a tiled GEMM: its configuration's, or 128 rows x 128 weight
+// rows -- deep: one workgroup per CU with a long ring; dual: two per CU.
+enum : int { kTileByConfig = 0, kTileDeep = 1, kTileDual = 2 };
+
 struct GemmParams {
   const uint8_t* a;
   const float* a_scale;   // fp8: [rows, kdim/128]; int8: [rows]; else null
@@ -73,6 +77,7 @@ struct GemmParams {
                               // and recorded in route_ids[j] for GEMM2 and
                               // the top-k sum; null: off
   int32_t* route_ids;
+  int32_t shape;              // tiled: the tile shape (kTileByConfig, ...)
 };
 
 // Router gating (scores -> top-k -> renormalise), one wave per token;
@@ -173,7 +178,9 @@ int launch_gemm2_pair(int dt, const GemmParams& p, int kw, hipStream_t stream);
 // 128 (GEMM2's 256-column tiles may end in a half tile).
 constexpr int kTiledConfigs = 5;  // row blocks 256, 128, 64, 32, 160
 int tiled_config_supported(int dt, int cfg);
-int tiled_config_for(int dt, double rows_per_expert, int num_experts);
+int tiled_config_for(int dt, double rows_per_expert, int num_experts, double tiles256,
+                     double tiles128);
+bool tile_forced();  // FGS_MOE_TILE is set
 int tiled_block_m(int cfg);
 int launch_gemm_tiled(int dt, int cfg, bool gemm1, const GemmParams& p,
                       int row_blocks, hipStream_t stream);

@@ -19,6 +19,7 @@
 // fp32 partial sums per split that moe_sum adds in a fixed order.
 #include <stdlib.h>
 
+#include <cmath>
 #include <mutex>
 #include <string>
 #include <type_traits>
@@ -75,9 +76,11 @@ __device__ __forceinline__ bool tile_of(int pid, int n_rb, int n_ct, int group_m
 // BMA < BM: a second, compact LDS ring for row blocks whose rows from BMA on
 // are all padding -- BMA activation rows per stage in STAGES_C slots (more
 // stages in flight than the full ring fits); fuller blocks use the full one.
+// WPE: waves per SIMD the register budget must leave room for.
 template <int BM_, int BNR_, int WM_, int WN_, int SK_, int STAGES_, int BMA_ = BM_,
-          int STAGES_C_ = STAGES_>
+          int STAGES_C_ = STAGES_, int WPE_ = 1>
 struct TileCfg {
+  static constexpr int WPE = WPE_;
   static constexpr int BM = BM_;        // rows (alignment block size)
   static constexpr int BNR = BNR_;      // weight rows per tile
   static constexpr int WM = WM_, WN = WN_;
@@ -873,7 +876,7 @@ __device__ __forceinline__ void tiled_tile(const GemmParams& p, const int rb_id,
 }
 
 template <int DT, class C, bool GEMM1>
-__global__ __launch_bounds__(C::NW * 64, 1) void moe_gemm_tiled_kernel(
+__global__ __launch_bounds__(C::NW * 64, C::WPE) void moe_gemm_tiled_kernel(
     const GemmParams p) {
   constexpr int BM = C::BM, BNR = C::BNR;
 
@@ -982,6 +985,17 @@ using Fp8Cfg256 = TileCfg<256, 128, 4, 2, 128, 3, 160, 4>;  // 8 waves of 64x64
 using Fp8Cfg64 = TileCfg<64, 256, 1, 4, 128, 3>;
 using Fp8Cfg32 = TileCfg<32, 256, 1, 4, 128, 3>;
 
+// 128 rows x 128 weight rows. Deep: grids of less than a round of workgroups,
+// where a CU's one tile waits for its own loads: 8 waves of 32x64 and 5 slots
+// of 32 KiB (fp8's scale area leaves 4), three or four stages in flight
+// (measured against 2 slots: hidden 4480, intermediate 896, 8 experts, 142
+// rows, layer 102 -> 88 us). Dual: two workgroups per CU of 4 waves of 64x64
+// (two slots, 256 registers a wave), which hide each other's prologue and
+// epilogue.
+using DeepCfg = TileCfg<128, 128, 4, 2, 128, 5>;
+using Fp8DeepCfg = TileCfg<128, 128, 4, 2, 128, 4>;
+using Fp8DualCfg = TileCfg<128, 128, 2, 2, 128, 2, 128, 2, 2>;
+
 static const int kTileRows[kTiledConfigs] = {Cfg256::BM, Cfg128::BM, Cfg64::BM,
                                              Cfg32::BM, Cfg160::BM};
 
@@ -1001,35 +1015,47 @@ int tiled_config_supported(int dt, int cfg) {
   return cfg >= 0 && cfg < kTiledConfigs;
 }
 
-// Configuration by rows per expert and expert count (measured on the four
-// model shapes, M from 32 to 8192):
-// * from 112 rows, 256-row blocks: fewer would spill a noticeable share of
-//   the experts into a second, mostly empty block that streams the
-//   expert's weights again, and the 256-row kernels skip the MFMAs of their
-//   all-pad 32-row blocks;
-// * with many experts (>= 32) the 256-row configuration already wins from
-//   48 rows (64 rows: Qwen3 -14 %, Qwen2 int8 -15 %, DeepSeek fp8 -10 %
-//   against the 64-row kernel); with 8 experts (Mixtral) it loses there;
-// * otherwise the 8-wave 128-row kernel from 24 rows (Mixtral M=256 -11 %,
-//   Qwen2 M=256 -6 %, DeepSeek M=1024 -4 %), and for many experts also from
-//   8 rows (Qwen2 M=64 -6 %, DeepSeek M=256/512 -3/-5 %, Qwen3 M=256 -7 %);
-// * the 32-row kernel below that (Mixtral M=32/64, DeepSeek M=32);
-// * bf16 with few experts takes the 256-row configuration from 96 rows
-//   (Mixtral M=384 -1.5 %, 448 -4 %, 512 -3.5 %, 576 -10 %, 640 -3.5 %
-//   against the 160-row kernel that had those rows; M=256, 64 rows, stays
-//   on the 128-row kernel: +5 % on 256-row blocks).
-// The 64- and 160-row configurations are no longer chosen; they stay for
+// Configuration by rows per expert and expert count. `tiles256`, `tiles128`:
+// the expected GEMM1 tiles (128 output columns) over 256- and 128-row blocks.
+// Layer time, us, 256- / 128-row blocks, weights rotated through more memory
+// than the caches, both forced:
+// * 256-row blocks from 112 rows per expert (fp8 122): from there a
+//   noticeable share of the experts would spill into a second, mostly empty
+//   128-row block that streams their weights again. Below, the 8-wave 128-row
+//   kernel: bf16 at 90 rows 339 / 321 (128 experts of 768), 722 / 686 (64 of
+//   2560), 367 / 346 (32 of 2944), 1555 / 1492 (160 of 1536), at 100 rows 753
+//   / 702 (64 of 2560), 110 rows 758 / 748, 120 rows 767 / 806; Mixtral 96
+//   rows 578 / 560, 112 rows 571 / 575; int8 at 90 rows 219 / 202, 452 / 420,
+//   249 / 226, 967 / 896, at 120 rows 480 / 491; fp8 237 / 205, 476 / 426,
+//   243 / 225, 1012 / 925, at 120 rows 530 / 522 (64 of 2560), 568 / 547 (of
+//   5888), DeepSeek 96 rows 2729 / 2520, 128 rows 3067 / 3227;
+// * on up to two rounds of CUs, the configuration of fewer rounds, a round
+//   of 256-row tiles counted as 1.45 (int8 1.65) rounds of 128-row ones
+//   (bf16 8 experts of 1792: 180 rows, one round each, 139 / 112; 512 rows,
+//   two each, 268 / 234; 256 rows, one and two, 153 / 174; 768 rows, two and
+//   three, 308 / 338; int8 107 / 85, 196 / 163, 116 / 124, 232 / 220);
+// * the 128-row kernel down to 24 rows, and with many experts (>= 32) to 8
+//   (Mixtral M=256, Qwen2 M=64, DeepSeek M=256, Qwen3 M=256 3..11 % faster
+//   than the 64- and 32-row ones);
+// * the 32-row kernel below that (Mixtral M=32/64, DeepSeek M=32).
+// The 64- and 160-row configurations are not chosen; they stay for
 // FGS_MOE_TILE.
-int tiled_config_for(int dt, double rows_per_expert, int num_experts) {
+int tiled_config_for(int dt, double rows_per_expert, int num_experts, double tiles256,
+                     double tiles128) {
   const bool many = num_experts >= 32;
   int c = 3;
-  if (rows_per_expert >= 112 || (many && rows_per_expert >= 48) ||
-      (dt == kDtBf16 && rows_per_expert >= 96))
-    c = 0;
-  else if (rows_per_expert >= 24 || (many && rows_per_expert >= 8)) c = 1;
+  if (rows_per_expert >= (dt == kDtFp8 ? 122 : 112)) {
+    const bool small = dt != kDtFp8 && tiles256 <= 2 * 256;
+    const double round256 = dt == kDtInt8 ? 1.65 : 1.45;
+    c = small && round256 * std::ceil(tiles256 / 256) > std::ceil(tiles128 / 256) ? 1 : 0;
+  } else if (rows_per_expert >= 24 || (many && rows_per_expert >= 8)) {
+    c = 1;
+  }
   if (forced_tile() >= 0) c = forced_tile();
   return c;
 }
+
+bool tile_forced() { return forced_tile() >= 0; }
 
 int tiled_block_m(int cfg) { return kTileRows[cfg]; }
 
@@ -1043,7 +1069,7 @@ static int launch_cfg(bool gemm1, const GemmParams& p, int row_blocks,
 void tiled_plan_request(int dt, int cfg, bool gemm1, const GemmParams& p, int row_blocks,
                         WidePlanReq* req) {
   *req = WidePlanReq{};
-  if (tiled_config_supported(dt, cfg) && row_blocks > 0 && cfg == 0 && wide_choice() >= 1 &&
+  if (tiled_config_supported(dt, cfg) && row_blocks > 0 && cfg == 0 && p.shape == kTileByConfig && wide_choice() >= 1 &&
       wide_supported(dt, gemm1, p))
     wide_plan_request(gemm1, p, row_blocks, req);
 }
@@ -1054,6 +1080,15 @@ int launch_gemm_tiled(int dt, int cfg, bool gemm1, const GemmParams& p,
     return fail(FGS_EINVAL, "tiled GEMM: configuration " + std::to_string(cfg) +
                                 " not available for this element type");
   if (row_blocks <= 0) return FGS_OK;
+  if (p.shape == kTileDeep) {
+    switch (dt) {
+      case kDtBf16: return launch_cfg<kDtBf16, DeepCfg>(gemm1, p, row_blocks, stream);
+      case kDtInt8: return launch_cfg<kDtInt8, DeepCfg>(gemm1, p, row_blocks, stream);
+      default: return launch_cfg<kDtFp8, Fp8DeepCfg>(gemm1, p, row_blocks, stream);
+    }
+  }
+  if (p.shape == kTileDual && dt == kDtFp8 && gemm1)
+    return launch_tiled<kDtFp8, Fp8DualCfg, true>(p, row_blocks, stream);
   // The 4-wave kernel runs both GEMMs of the 256-row configuration: with
   // its weight rows a stage ahead it also wins on the long GEMM2
   // contraction it used to leave to the 8-wave kernel (Mixtral, 28 KiB k

@@ -38,26 +38,39 @@ def test_odd_hidden_tiled_configs(gpu, mode, K, N):
         assert torch.equal(outs[0], outs[cfg]), f"{mode} K={K} N={N}: tile 0 vs tile {cfg}"
 
 
-# (2100, 4224, ...): 1 to 8 rounds of tiles, the split tail; (700, 1408, ...):
-# a k split of 128-row tiles; the default schedule of each
-@pytest.mark.parametrize("shape", [(2100, 4224, 512, 8, 2), (700, 1408, 2048, 16, 1)])
+def _within_ulps(res, ref):
+    """Against the oracle, in bf16 ulps of the summed terms' magnitude: sums in
+    another order may round each slot's row (together at most one ulp of the
+    magnitude) and the result (one more) to the neighbouring value, and an
+    intermediate element with them (well under another). Over the ~200k
+    outputs compared here both do at once now and then, and two ulps are up to
+    1.6 % of the magnitude, past the elementwise tolerance of 1 %."""
+    st = testing.regression_stats(res, *ref)
+    assert st["max_ulp_mag"] <= 4 and st["mean_rel"] <= 1e-3, st
+
+
+# the split tail on half tiles (1 to 8 rounds of tiles, 40 stages of k) and a
+# k split of them
+@pytest.mark.parametrize("shape", [(2100, 4224, 3200, 8, 2), (128, 4224, 2560, 8, 2)])
 def test_odd_hidden_splits(gpu, shape):
     M, K, N, E, topk = shape
+    sched = _capi.schedule(M, K, N, E, topk, _capi.QMODE_BF16)
+    assert "tail2" in sched or "ksplit2" in sched, sched
     x, w1, w2, b1, b2, w, ids = _bias_inputs(M, K, N, E, topk, gpu)
     toks = _sample(M, 48)
     res = fm.fused_moe(x, w1, w2, w, ids)
     ref = moe_ref.fused_moe(x, w1, w2, w, ids, tokens=toks, return_mag=True)
-    _check(res.cpu()[toks], ref, "bf16", f"odd hidden {shape}")
+    _within_ulps(res.cpu()[toks], ref)
     res = fm.fused_moe_with_bias(x, w1, b1, w2, b2, w, ids, interleaved=False)
     ref = moe_ref.fused_moe(x, w1, w2, w, ids, tokens=toks, return_mag=True,
                             activation="swiglu", b1=b1, b2=b2)
-    _check(res.cpu()[toks], ref, "bf16", f"odd hidden bias {shape}")
+    _within_ulps(res.cpu()[toks], ref)
 
 
 def test_odd_hidden_no_alloc_streams(gpu):
     """The tiled schedule's split-tail workspace alone is the whole device
     scratch; the streaming one fits, and the call is still served."""
-    M, K, N, E, topk = 2048, 4224, 256, 8, 2
+    M, K, N, E, topk = 2100, 4224, 3200, 8, 2
     wts = testing.make_weights(K, N, E, "bf16", 0.05, device=gpu, seed=K)
     x, w, ids = testing.make_tokens(M, K, E, topk, device=gpu)
     out = _no_alloc(x, wts.w1, wts.w2, w, ids)
@@ -100,3 +113,49 @@ def test_wide_activations(gpu, act, mode, on_input):
     _check(out.cpu(), ref, mode, f"wide {act} {mode} {on_input}")
     for cfg in (1, 3):
         assert torch.equal(out, run(cfg)), f"{act} {mode}: tile 0 vs tile {cfg}"
+
+
+_QM = {"bf16": _capi.QMODE_BF16, "fp8": _capi.QMODE_FP8_BLOCK, "int8": _capi.QMODE_INT8_CHANNEL}
+_SCHEDULED = [
+    # 128x128 tiles, one per CU: k rows of one or two stages, of less and of
+    # more than the ring, the last block of an expert partly filled
+    ("bf16", (60, 128, 128, 4, 2), "deep1 deep2"),
+    ("bf16", (61, 384, 256, 4, 2), "deep1 deep2"),
+    ("bf16", (700, 1152, 640, 4, 2), "deep1 deep2"),
+    ("int8", (60, 256, 256, 4, 2), "deep1 deep2"),
+    ("int8", (500, 1280, 768, 4, 2), "deep1 deep2"),
+    ("fp8", (60, 128, 128, 4, 2), "deep1 deep2"),
+    ("fp8", (333, 896, 640, 4, 2), "deep1 deep2"),
+    # fp8 GEMM1 two workgroups per CU on halves of 256-row blocks
+    ("fp8", (1700, 128, 1024, 32, 4), "dual1"),
+    ("fp8", (1801, 384, 1152, 32, 4), "dual1"),
+    # fp8 GEMM2 on the 160-row ring
+    ("fp8", (1050, 384, 2560, 16, 2), "cfg=0 cfg2=0"),
+    # the split tail, a k split
+    ("bf16", (2600, 1152, 2560, 32, 2), "tail2"),
+    ("int8", (2600, 1280, 5120, 32, 2), "tail2"),
+    ("bf16", (128, 4096, 4096, 8, 2), "cfg2=1 ksplit2=2"),
+    ("bf16", (128, 1280, 4096, 8, 2), "deep2 ksplit2=3"),
+]
+
+
+@pytest.mark.parametrize("mode,shape,expect", _SCHEDULED,
+                         ids=[f"{m}-{s}-{e}".replace(" ", "") for m, s, e in _SCHEDULED])
+def test_scheduled_shapes(gpu, mode, shape, expect):
+    """What the schedule's rules pick off the benchmarked sizes, against the
+    oracle and (tiled) bit for bit against the 128-row configuration."""
+    M, K, N, E, topk = shape
+    sched = _capi.schedule(M, K, N, E, topk, _QM[mode])
+    assert expect in sched, sched
+    wts = testing.make_weights(K, N, E, mode, 0.05, device=gpu, seed=M + K + N)
+    x, w, ids = testing.make_tokens(M, K, E, topk, device=gpu, seed=M + K + N)
+    res = fm.fused_moe(x, wts.w1, wts.w2, w, ids, **wts.kwargs(mode))
+    toks = _sample(M, 48)
+    ref = moe_ref.fused_moe(x, wts.w1, wts.w2, w, ids, mode=mode, w1_scale=wts.w1_scale,
+                            w2_scale=wts.w2_scale, tokens=toks, return_mag=True)
+    _check(res.cpu()[toks], ref, mode, f"{sched} {shape} {mode}",
+           ulp_mag=8.0 if mode == "fp8" else None)
+    if ("deep" in sched or "dual" in sched) and "ksplit" not in sched:
+        other = fm.fused_moe(x, wts.w1, wts.w2, w, ids, _flags=_capi.flag_tile(1),
+                             **wts.kwargs(mode))
+        assert torch.equal(res, other)

@@ -53,6 +53,13 @@ __device__ __forceinline__ void align_write_plans(int lane, const int32_t* off,
                     r1.plan);
 }
 
+// The class an id sorts under: itself inside [0, num_classes), else `other`
+// (-1: the slot is dropped). Where `other` is a class, the kernels write the
+// counts of the classes below it to `hist` when it is given.
+__device__ __forceinline__ int class_of(int id, int num_classes, int other) {
+  return id >= 0 && id < num_classes ? id : other;
+}
+
 constexpr int kAlignWaves = 16;
 constexpr int64_t kAlignMultiMin = 4096;  // slots from which the multi-WG path runs
 constexpr int kAlignThreads = kAlignWaves * kWave;
@@ -61,7 +68,8 @@ __global__ __launch_bounds__(kAlignThreads) void moe_align_kernel(
     const int32_t* __restrict__ ids, int64_t numel, int num_experts,
     int block_size, int id_bits, int32_t* __restrict__ sorted_ids,
     int32_t* __restrict__ expert_ids, int32_t* __restrict__ num_post_pad,
-    int64_t max_padded, WidePlanReq plan0, WidePlanReq plan1) {
+    int64_t max_padded, WidePlanReq plan0, WidePlanReq plan1, int other,
+    int32_t* __restrict__ hist) {
   // cnt[w * E + e]: pass 1 count, then (after pass 2) the slot cursor.
   extern __shared__ int32_t smem[];
   int32_t* cnt = smem;                                  // [16][E]
@@ -85,8 +93,8 @@ __global__ __launch_bounds__(kAlignThreads) void moe_align_kernel(
 
   // Pass 1: per-(wave, expert) histogram.
   for (int64_t i = beg + lane; i < end; i += kWave) {
-    const int e = ids[i];
-    if (e >= 0 && e < E) atomicAdd(&cnt[wave * E + e], 1);
+    const int e = class_of(ids[i], E, other);
+    if (e >= 0) atomicAdd(&cnt[wave * E + e], 1);
   }
   __syncthreads();
 
@@ -99,6 +107,7 @@ __global__ __launch_bounds__(kAlignThreads) void moe_align_kernel(
       run += c;
     }
     tot[e] = run;
+    if (hist && e < other && blockIdx.x == 0) hist[e] = run;
   }
   __syncthreads();
 
@@ -162,11 +171,7 @@ __global__ __launch_bounds__(kAlignThreads) void moe_align_kernel(
   const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (kWave - lane));
   for (int64_t c0 = beg; c0 < end; c0 += kWave) {
     const int64_t i = c0 + lane;
-    int e = -1;
-    if (i < end) {
-      e = ids[i];
-      if (e < 0 || e >= E) e = -1;
-    }
+    const int e = i < end ? class_of(ids[i], E, other) : -1;
     const bool valid = e >= 0;
     uint64_t match = __ballot(valid);
     for (int b = 0; b < id_bits; ++b) {
@@ -203,15 +208,15 @@ constexpr int kChunk = 1024;  // slots per chunk (256 per wave)
 
 __global__ __launch_bounds__(kChunkThreads) void moe_align_count_kernel(
     const int32_t* __restrict__ ids, int64_t numel, int num_experts,
-    int32_t* __restrict__ counts) {
+    int32_t* __restrict__ counts, int other) {
   extern __shared__ int32_t hist[];  // [E]
   const int E = num_experts;
   for (int e = threadIdx.x; e < E; e += kChunkThreads) hist[e] = 0;
   __syncthreads();
   const int64_t c0 = static_cast<int64_t>(blockIdx.x) * kChunk;
   for (int64_t i = c0 + threadIdx.x; i < c0 + kChunk && i < numel; i += kChunkThreads) {
-    const int e = ids[i];
-    if (e >= 0 && e < E) atomicAdd(&hist[e], 1);
+    const int e = class_of(ids[i], E, other);
+    if (e >= 0) atomicAdd(&hist[e], 1);
   }
   __syncthreads();
   for (int e = threadIdx.x; e < E; e += kChunkThreads)
@@ -223,7 +228,7 @@ __global__ __launch_bounds__(kChunkThreads) void moe_align_scatter_kernel(
     int block_size, int id_bits, const int32_t* __restrict__ counts,
     int32_t* __restrict__ sorted_ids, int32_t* __restrict__ expert_ids,
     int32_t* __restrict__ num_post_pad, int64_t max_padded, WidePlanReq plan0,
-    WidePlanReq plan1) {
+    WidePlanReq plan1, int other, int32_t* __restrict__ hist) {
   extern __shared__ int32_t smem[];
   const int E = num_experts;
   int32_t* cnt = smem;                         // [4][E]: wave counts, then cursors
@@ -259,6 +264,7 @@ __global__ __launch_bounds__(kChunkThreads) void moe_align_scatter_kernel(
     }
     pre[e] = before;
     tot[e] = all;
+    if (hist && e < other && c == 0) hist[e] = all;
   }
   for (int i = tid; i < kChunkWaves * E; i += kChunkThreads) cnt[i] = 0;
   __syncthreads();
@@ -298,8 +304,8 @@ __global__ __launch_bounds__(kChunkThreads) void moe_align_scatter_kernel(
   const int64_t wbeg = static_cast<int64_t>(c) * kChunk + wave * (kChunk / kChunkWaves);
   const int64_t wend = wbeg + kChunk / kChunkWaves < numel ? wbeg + kChunk / kChunkWaves : numel;
   for (int64_t i = wbeg + lane; i < wend; i += kWave) {
-    const int e = ids[i];
-    if (e >= 0 && e < E) atomicAdd(&cnt[wave * E + e], 1);
+    const int e = class_of(ids[i], E, other);
+    if (e >= 0) atomicAdd(&cnt[wave * E + e], 1);
   }
   __syncthreads();
   // cursors: expert offset + earlier chunks + earlier waves of this chunk
@@ -333,11 +339,7 @@ __global__ __launch_bounds__(kChunkThreads) void moe_align_scatter_kernel(
   const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (kWave - lane));
   for (int64_t c0 = wbeg; c0 < wend; c0 += kWave) {
     const int64_t i = c0 + lane;
-    int e = -1;
-    if (i < wend) {
-      e = ids[i];
-      if (e < 0 || e >= E) e = -1;
-    }
+    const int e = i < wend ? class_of(ids[i], E, other) : -1;
     const bool valid = e >= 0;
     uint64_t match = __ballot(valid);
     for (int b = 0; b < id_bits; ++b) {
@@ -375,13 +377,10 @@ int64_t align_scratch_bytes(int64_t numel, int num_experts) {
 __global__ __launch_bounds__(kWave) void moe_align_wave_kernel(
     const int32_t* __restrict__ ids, int numel, int num_experts, int block_size,
     int id_bits, int32_t* __restrict__ sorted_ids, int32_t* __restrict__ expert_ids,
-    int32_t* __restrict__ num_post_pad, int64_t max_padded) {
+    int32_t* __restrict__ num_post_pad, int64_t max_padded, int other,
+    int32_t* __restrict__ hist) {
   const int lane = threadIdx.x;
-  int e = -1;
-  if (lane < numel) {
-    e = ids[lane];
-    if (e < 0 || e >= num_experts) e = -1;  // dropped slot
-  }
+  const int e = lane < numel ? class_of(ids[lane], num_experts, other) : -1;
   const bool valid = e >= 0;
   uint64_t eq = __ballot(valid);
   uint64_t lt = 0;
@@ -404,7 +403,10 @@ __global__ __launch_bounds__(kWave) void moe_align_wave_kernel(
     total += __popcll(pk) << k;
   }
   for (int64_t q = lane; q < max_padded; q += kWave) sorted_ids[q] = numel;
-  __builtin_amdgcn_s_waitcnt(0);  // the sentinel fill completes before the slots
+  if (hist)
+    for (int q = lane; q < other; q += kWave) hist[q] = 0;
+  __builtin_amdgcn_s_waitcnt(0);  // the fills complete before the slots and counts
+  if (hist && first && e < other) hist[e] = cnt;
   if (valid) sorted_ids[off + rank] = lane;
   if (first)
     for (int blk = off / block_size; blk < (off + cnt + pad) / block_size; ++blk)
@@ -423,7 +425,7 @@ int launch_align(const int32_t* ids, int64_t numel, int num_experts,
                  int block_size, int32_t* sorted_ids, int32_t* expert_ids,
                  int32_t* num_post_pad, int64_t max_padded,
                  hipStream_t stream, int32_t* scratch, const WidePlanReq* plans,
-                 bool* planned) {
+                 bool* planned, int other, int32_t* hist) {
   int id_bits = 0;
   while ((1 << id_bits) < num_experts) ++id_bits;
   WidePlanReq plan0{}, plan1{};
@@ -435,7 +437,7 @@ int launch_align(const int32_t* ids, int64_t numel, int num_experts,
   if (numel <= kWave) {
     hipLaunchKernelGGL(moe_align_wave_kernel, dim3(1), dim3(kWave), 0, stream, ids,
                        static_cast<int>(numel), num_experts, block_size, id_bits,
-                       sorted_ids, expert_ids, num_post_pad, max_padded);
+                       sorted_ids, expert_ids, num_post_pad, max_padded, other, hist);
     return check_launch("moe_align_wave_kernel");
   }
   if (scratch && numel >= kAlignMultiMin) {
@@ -443,14 +445,15 @@ int launch_align(const int32_t* ids, int64_t numel, int num_experts,
     const size_t smem1 = sizeof(int32_t) * num_experts;
     const size_t smem2 = sizeof(int32_t) * ((kChunkWaves + 3) * num_experts + 1);
     hipLaunchKernelGGL(moe_align_count_kernel, dim3(nchunks), dim3(kChunkThreads),
-                       smem1, stream, ids, numel, num_experts, scratch);
+                       smem1, stream, ids, numel, num_experts, scratch, other);
     int rc = check_launch("moe_align_count_kernel");
     if (rc) return rc;
     const bool with_plans = plan0.plan || plan1.plan;
     hipLaunchKernelGGL(moe_align_scatter_kernel, dim3(nchunks + (with_plans ? 1 : 0)),
                        dim3(kChunkThreads),
                        smem2, stream, ids, numel, num_experts, block_size, id_bits,
-                       scratch, sorted_ids, expert_ids, num_post_pad, max_padded, plan0, plan1);
+                       scratch, sorted_ids, expert_ids, num_post_pad, max_padded, plan0, plan1, other,
+                       hist);
     rc = check_launch("moe_align_scatter_kernel");
     if (!rc && planned) *planned = plan0.plan || plan1.plan;
     return rc;
@@ -473,7 +476,7 @@ int launch_align(const int32_t* ids, int64_t numel, int num_experts,
   const bool with_plans = plan0.plan || plan1.plan;
   hipLaunchKernelGGL(moe_align_kernel, dim3(with_plans ? 2 : 1), dim3(kAlignThreads), smem,
                      stream, ids, numel, num_experts, block_size, id_bits,
-                     sorted_ids, expert_ids, num_post_pad, max_padded, plan0, plan1);
+                     sorted_ids, expert_ids, num_post_pad, max_padded, plan0, plan1, other, hist);
   const int rc = check_launch("moe_align_kernel");
   if (!rc && planned) *planned = plan0.plan || plan1.plan;
   return rc;

@@ -95,12 +95,14 @@ int64_t align_scratch_bytes(int64_t numel, int num_experts);
 // workgroups; without it, one workgroup. Same output either way.
 // `plans` (two requests, or null): the 4-wave GEMMs' tile plans, written
 // from the per-expert counts by the same launch; *planned says whether they
-// were (not on the single-wave path for at most 64 slots).
+// were (not on the single-wave path for at most 64 slots). `other`: the
+// class of ids outside [0, num_experts) (-1: dropped); `hist` (or null): the
+// counts of the classes below `other`.
 int launch_align(const int32_t* ids, int64_t numel, int num_experts,
                  int block_size, int32_t* sorted_ids, int32_t* expert_ids,
                  int32_t* num_post_pad, int64_t max_padded, hipStream_t stream,
                  int32_t* scratch = nullptr, const WidePlanReq* plans = nullptr,
-                 bool* planned = nullptr);
+                 bool* planned = nullptr, int other = -1, int32_t* hist = nullptr);
 
 // Routing-format conversion (routing.hip): the triton_kernels routing tuple
 // of _standard_topk_to_triton_kernels, block metadata for block_m in

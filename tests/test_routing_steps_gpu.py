@@ -30,3 +30,59 @@ def test_gating_ranks(gpu, E, scoring):
     assert torch.equal(ids.cpu(), rids)
     # a score: the exponential's and the sum's fp32 rounding (2 ulps each)
     assert torch.allclose(w.cpu(), rw, rtol=2e-6, atol=1e-7)
+
+
+@pytest.mark.parametrize("M,k,E", [(0, 4, 65), (8, 8, 64), (9, 8, 65), (64, 4, 128),
+                                   (512, 8, 129), (513, 8, 256), (700, 6, 1022), (3, 1, 1)])
+def test_conversion_tables(gpu, M, k, E):
+    """One, 64, 65, 4095.. slots and whole and partial waves of experts: the
+    single-wave, single- and many-workgroup alignments write the histogram,
+    the last workgroup of the finishing launch the tables. Ids on either side
+    of [0, E) sort behind the experts and count for none."""
+    g = torch.Generator().manual_seed(M + E)
+    ids = torch.stack([torch.randperm(E, generator=g)[:k] for _ in range(M)]).int() if M else \
+        torch.empty(0, k, dtype=torch.int32)
+    ids[::3, -1] = -1
+    ids[1::5, 0] = E
+    ids[2::5, 0] = 2 ** 30
+    w = torch.rand(M, k, generator=g)
+    rd, gi, si = fm.standard_topk_to_routing(w.to(gpu), ids.to(gpu), E)
+    # the oracle's dropped id is -1
+    known = torch.where((ids >= 0) & (ids < E), ids, torch.full_like(ids, -1))
+    hist = torch.bincount(known[known >= 0].long().reshape(-1), minlength=E).int()
+    assert torch.equal(rd.expt_hist.cpu(), hist)
+    raw, pad, pid = moe_ref.expt_data(hist.numpy(), E, M * k)
+    assert torch.equal(rd.expt_data.token_offs_raw.cpu(), torch.from_numpy(raw))
+    for bm in moe_ref.ROUTING_BLOCK_MS:
+        assert torch.equal(rd.expt_data.token_offs_pad[bm].cpu(), torch.from_numpy(pad[bm]))
+        assert torch.equal(rd.expt_data.block_pid_map[bm].cpu(), torch.from_numpy(pid[bm]))
+    # every expert's range of the gathered order holds its slots, in slot order
+    rank = torch.argsort(ids, dim=1, stable=True)            # slot of each row-sorted place
+    slot = (rank + torch.arange(M)[:, None] * k).reshape(-1)
+    src = gi.src_indx.cpu().long()
+    got = known.reshape(-1)[slot[src]] if M else src
+    n = int(hist.sum())
+    assert torch.equal(got[:n], torch.repeat_interleave(torch.arange(E), hist.long()).int())
+    assert bool((got[n:] == -1).all())
+    for e in range(E):
+        assert bool((slot[src[raw[e]:raw[e + 1]]].diff() > 0).all())
+    assert torch.equal(si.src_indx.cpu().long()[src], torch.arange(M * k))
+    assert torch.equal(rd.gate_scal.cpu(), w.reshape(-1)[slot[src]] if M else w.reshape(-1))
+
+
+@pytest.mark.parametrize("E", [1, 64, 65, 130, 1024])
+def test_order_from_extreme_histograms(gpu, E):
+    """Counts of a caller's histogram up to the type's limits: the running
+    sums are cut at the gate count without wrapping in 32 bits."""
+    n = 3 * E
+    hist = torch.full((E,), 2 ** 31 - 1, dtype=torch.int32)
+    hist[::2] = -(2 ** 31)
+    hist[0] = 2
+    g = torch.Generator().manual_seed(E)
+    src = torch.randperm(n, generator=g).int()
+    gs = torch.rand(n, generator=g)
+    _, _, _, rid, rwt = moe_ref.routing_order(gs.numpy(), src.numpy(), hist.numpy(), n, 1)
+    tw, ti = fm._routing_to_topk(fm.RoutingData(gs.to(gpu), hist.to(gpu), E, 3),
+                                 fm.GatherIndx(src.to(gpu), src.to(gpu)), E)
+    assert torch.equal(ti.cpu().reshape(-1), torch.from_numpy(rid))
+    assert torch.equal(tw.cpu().reshape(-1), torch.from_numpy(rwt))

@@ -16,6 +16,7 @@ Reference interface mirrored: src/flaggems_sglang/ops/fused_moe.py
 from __future__ import annotations
 
 import logging
+import sys
 import weakref
 from dataclasses import dataclass
 from typing import Optional
@@ -30,7 +31,15 @@ logger = logging.getLogger(__name__)
 _UNSUPPORTED_FEATURE_MSG = "{name} is not supported"
 
 
+# torch's current HIP stream of a device index as an integer: the accessor
+# torch's own generated code uses (0.1 us; building a Stream object for its
+# handle takes 1.9), or that object where torch lacks it
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream_ptr(t: torch.Tensor) -> int:
+    if _raw_stream is not None:
+        return _raw_stream(t.get_device())
     return torch.cuda.current_stream(t.device).cuda_stream
 
 
@@ -60,14 +69,20 @@ class _ConversionCache:
     once -- and never a copy of a dead one. A conversion that returns a view
     of its source (a transposed view that is already contiguous in the other
     order) costs nothing and is not stored: storing it would keep the root
-    alive.
+    alive. ``view``: the conversion as a view, which is the result where it
+    is contiguous (taken before any lookup).
     """
 
-    def __init__(self, fn):
+    def __init__(self, fn, view=None):
         self._fn = fn
+        self._view = view
         self._roots: dict = {}  # id(root) -> {geometry: (version, converted)}
 
     def __call__(self, w: torch.Tensor) -> torch.Tensor:
+        if self._view is not None:
+            v = self._view(w)
+            if v.is_contiguous():
+                return v
         root = w._base if w._base is not None else w
         geometry = (w.storage_offset(), tuple(w.shape), tuple(w.stride()), w.dtype)
         stamp = (root._version, root.untyped_storage().data_ptr())
@@ -184,9 +199,10 @@ def standard_topk_to_routing(topk_weights, topk_ids, n_expts_tot):
         "standard_topk_to_routing",
     )
     bms = _capi.ROUTING_BLOCK_MS
-    expt = ExptData(hist, offs_raw,
-                    {bm: offs_pad[i] for i, bm in enumerate(bms)},
-                    {bm: pid_map[i, :max_tiles] for i, bm in enumerate(bms)})
+    if max_tiles == 0:
+        pid_map = pid_map[:, :0]
+    expt = ExptData(hist, offs_raw, dict(zip(bms, offs_pad.unbind(0))),
+                    dict(zip(bms, pid_map.unbind(0))))
     routing = RoutingData(gate_scal, hist, E, k, expt)
     return (
         routing,
@@ -604,7 +620,8 @@ def _fused_routed(hidden_states, w1, w2, routing_data, gather_indx, *,
 # plugin transposes both weights on every call, ops/fused_moe.py:342-343).
 # A weight passed as a transposed view of a native-layout tensor converts
 # for free.
-_native_layout = _ConversionCache(lambda t: t.transpose(-1, -2).contiguous())
+_native_layout = _ConversionCache(lambda t: t.transpose(-1, -2).contiguous(),
+                                  view=lambda t: t.transpose(-1, -2))
 
 
 def clear_weight_cache() -> None:
@@ -912,14 +929,29 @@ class StandardCombineInput:
     hidden_states: torch.Tensor
 
 
+_combine_cls = None
+_sglang_absent = False
+
+
 def _combine_input_cls():
+    """SGLang's result type, or the stand-in where SGLang cannot be imported.
+    The import is tried once, and again only after something else has
+    imported SGLang (a failing import searches every path entry: ~40 us on
+    each call)."""
+    global _combine_cls, _sglang_absent
+    if _combine_cls is not None:
+        return _combine_cls
+    if _sglang_absent and "sglang" not in sys.modules:
+        return StandardCombineInput
     try:
         from sglang.srt.layers.moe.token_dispatcher.standard import (
             StandardCombineInput as cls,
         )
-        return cls
     except Exception:
+        _sglang_absent = True
         return StandardCombineInput
+    _combine_cls = cls
+    return cls
 
 
 def fused_moe_flagos(obj, layer, dispatch_output):

@@ -69,7 +69,7 @@ __global__ __launch_bounds__(kAlignThreads) void moe_align_kernel(
     int block_size, int id_bits, int32_t* __restrict__ sorted_ids,
     int32_t* __restrict__ expert_ids, int32_t* __restrict__ num_post_pad,
     int64_t max_padded, WidePlanReq plan0, WidePlanReq plan1, int other,
-    int32_t* __restrict__ hist) {
+    int32_t* __restrict__ hist, int32_t* __restrict__ slot_pos) {
   // cnt[w * E + e]: pass 1 count, then (after pass 2) the slot cursor.
   extern __shared__ int32_t smem[];
   int32_t* cnt = smem;                                  // [16][E]
@@ -184,6 +184,7 @@ __global__ __launch_bounds__(kAlignThreads) void moe_align_kernel(
     const int rank = __popcll(match & lt_mask);
     // Highest matching lane advances the cursor after every lane has read it.
     __builtin_amdgcn_wave_barrier();
+    if (slot_pos && i < end) slot_pos[i] = valid ? off[e] + base + rank : -1;
     if (valid) {
       sorted_ids[off[e] + base + rank] = static_cast<int32_t>(i);
       const bool leader = (match >> lane) == 1ull;
@@ -228,7 +229,8 @@ __global__ __launch_bounds__(kChunkThreads) void moe_align_scatter_kernel(
     int block_size, int id_bits, const int32_t* __restrict__ counts,
     int32_t* __restrict__ sorted_ids, int32_t* __restrict__ expert_ids,
     int32_t* __restrict__ num_post_pad, int64_t max_padded, WidePlanReq plan0,
-    WidePlanReq plan1, int other, int32_t* __restrict__ hist) {
+    WidePlanReq plan1, int other, int32_t* __restrict__ hist,
+    int32_t* __restrict__ slot_pos) {
   extern __shared__ int32_t smem[];
   const int E = num_experts;
   int32_t* cnt = smem;                         // [4][E]: wave counts, then cursors
@@ -351,6 +353,7 @@ __global__ __launch_bounds__(kChunkThreads) void moe_align_scatter_kernel(
     if (valid) base = cnt[wave * E + e];
     const int rank = __popcll(match & lt_mask);
     __builtin_amdgcn_wave_barrier();
+    if (slot_pos && i < wend) slot_pos[i] = valid ? base + rank : -1;
     if (valid) {
       sorted_ids[base + rank] = static_cast<int32_t>(i);
       const bool leader = (match >> lane) == 1ull;
@@ -378,7 +381,7 @@ __global__ __launch_bounds__(kWave) void moe_align_wave_kernel(
     const int32_t* __restrict__ ids, int numel, int num_experts, int block_size,
     int id_bits, int32_t* __restrict__ sorted_ids, int32_t* __restrict__ expert_ids,
     int32_t* __restrict__ num_post_pad, int64_t max_padded, int other,
-    int32_t* __restrict__ hist) {
+    int32_t* __restrict__ hist, int32_t* __restrict__ slot_pos) {
   const int lane = threadIdx.x;
   const int e = lane < numel ? class_of(ids[lane], num_experts, other) : -1;
   const bool valid = e >= 0;
@@ -408,6 +411,7 @@ __global__ __launch_bounds__(kWave) void moe_align_wave_kernel(
   __builtin_amdgcn_s_waitcnt(0);  // the fills complete before the slots and counts
   if (hist && first && e < other) hist[e] = cnt;
   if (valid) sorted_ids[off + rank] = lane;
+  if (slot_pos && lane < numel) slot_pos[lane] = valid ? off + rank : -1;
   if (first)
     for (int blk = off / block_size; blk < (off + cnt + pad) / block_size; ++blk)
       expert_ids[blk] = e;
@@ -425,7 +429,7 @@ int launch_align(const int32_t* ids, int64_t numel, int num_experts,
                  int block_size, int32_t* sorted_ids, int32_t* expert_ids,
                  int32_t* num_post_pad, int64_t max_padded,
                  hipStream_t stream, int32_t* scratch, const WidePlanReq* plans,
-                 bool* planned, int other, int32_t* hist) {
+                 bool* planned, int other, int32_t* hist, int32_t* slot_pos) {
   int id_bits = 0;
   while ((1 << id_bits) < num_experts) ++id_bits;
   WidePlanReq plan0{}, plan1{};
@@ -437,7 +441,7 @@ int launch_align(const int32_t* ids, int64_t numel, int num_experts,
   if (numel <= kWave) {
     hipLaunchKernelGGL(moe_align_wave_kernel, dim3(1), dim3(kWave), 0, stream, ids,
                        static_cast<int>(numel), num_experts, block_size, id_bits,
-                       sorted_ids, expert_ids, num_post_pad, max_padded, other, hist);
+                       sorted_ids, expert_ids, num_post_pad, max_padded, other, hist, slot_pos);
     return check_launch("moe_align_wave_kernel");
   }
   if (scratch && numel >= kAlignMultiMin) {
@@ -453,7 +457,7 @@ int launch_align(const int32_t* ids, int64_t numel, int num_experts,
                        dim3(kChunkThreads),
                        smem2, stream, ids, numel, num_experts, block_size, id_bits,
                        scratch, sorted_ids, expert_ids, num_post_pad, max_padded, plan0, plan1, other,
-                       hist);
+                       hist, slot_pos);
     rc = check_launch("moe_align_scatter_kernel");
     if (!rc && planned) *planned = plan0.plan || plan1.plan;
     return rc;
@@ -476,7 +480,8 @@ int launch_align(const int32_t* ids, int64_t numel, int num_experts,
   const bool with_plans = plan0.plan || plan1.plan;
   hipLaunchKernelGGL(moe_align_kernel, dim3(with_plans ? 2 : 1), dim3(kAlignThreads), smem,
                      stream, ids, numel, num_experts, block_size, id_bits,
-                     sorted_ids, expert_ids, num_post_pad, max_padded, plan0, plan1, other, hist);
+                     sorted_ids, expert_ids, num_post_pad, max_padded, plan0, plan1, other, hist,
+                     slot_pos);
   const int rc = check_launch("moe_align_kernel");
   if (!rc && planned) *planned = plan0.plan || plan1.plan;
   return rc;

@@ -80,7 +80,7 @@ struct Plan {
   int64_t max_padded, n_blocks, n_launch;
   // workspace layout (byte offsets)
   int64_t o_sorted, o_eids, o_npp, o_alg, o_a2, o_xq, o_xs, o_a2q, o_a2s, o_y, o_tail,
-      o_xst, o_rids, o_rw, o_plan, o_plan2,
+      o_xst, o_rids, o_rw, o_plan, o_plan2, o_pos,
       total;
 };
 
@@ -490,6 +490,7 @@ static int make_plan(int64_t m, int64_t hidden, int64_t inter, int e, int topk,
   // a call on the routing tuple: each flat slot's expert id and gate scale
   p.o_rids = take(numel * 4);
   p.o_rw = take(numel * 4);
+  p.o_pos = p.dt != kDtBf16 && !p.direct ? take(numel * 4) : -1;
   p.total = o;
   *pl = p;
   return FGS_OK;
@@ -743,9 +744,12 @@ static int run_fused(const FusedArgs& a) {
   g2.shape = p.shape2;
   const int rows2 = static_cast<int>(p.n_launch << p.eid_shift2);
 
+  // (quantised modes) each slot's row of the padded order, for the quantiser
+  // of the GEMM1 output
+  int32_t* slot_pos = p.o_pos >= 0 ? reinterpret_cast<int32_t*>(ws + p.o_pos) : nullptr;
   if (routed && !p.direct) {
     rc = launch_routing_order(a.gate_scal, a.gather_src, a.expt_hist, numel, a.e, p.block_m,
-                              p.max_padded, sorted, eids, npp, rids, rw, a.stream);
+                              p.max_padded, sorted, eids, npp, rids, rw, a.stream, slot_pos);
     if (rc) return rc;
   } else if (!p.direct) {
     // the alignment also writes the 4-wave GEMMs' tile plans (their launches
@@ -759,7 +763,7 @@ static int run_fused(const FusedArgs& a) {
     rc = launch_align(topk_ids, numel, a.e, p.block_m, sorted, eids, npp,
                       p.max_padded, a.stream,
                       p.o_alg >= 0 ? reinterpret_cast<int32_t*>(ws + p.o_alg) : nullptr,
-                      req, &planned);
+                      req, &planned, -1, nullptr, slot_pos);
     if (rc) return rc;
     g1.plan_ready = planned && req[0].plan ? 1 : 0;
     g2.plan_ready = planned && req[1].plan ? 1 : 0;
@@ -793,24 +797,20 @@ static int run_fused(const FusedArgs& a) {
   if (rc) return rc;
   g_prof.mark(3, a.stream);
 
-  // direct rows: the compact slot rows; else only the padded rows in use
-  // (num_tokens_post_padded, on the device)
-  const int64_t a2_rows = p.direct ? numel : p.max_padded;
-  const int32_t* a2_npp = p.direct ? nullptr : npp;
-  const int32_t* a2_sorted = p.direct ? nullptr : sorted;
+  // direct rows: the compact slot rows; else each slot's padded row
   if (p.qfold) {
     // GEMM2 quantises the a2 slot rows itself
   } else if (p.dt == kDtFp8) {
     // tiled: the scales k-block-major over the padded rows (see o_xst)
     rc = launch_quant_fp8_group(a2, ws + p.o_a2q,
                                 reinterpret_cast<float*>(ws + p.o_a2s),
-                                a2_rows, a.inter, 128, a.stream, a2_npp, a2_sorted, numel,
+                                numel, a.inter, 128, a.stream, slot_pos, p.max_padded,
                                 p.tiled ? p.max_padded : 0);
     if (rc) return rc;
   } else if (p.dt == kDtInt8) {
     rc = launch_quant_int8_token(a2, reinterpret_cast<int8_t*>(ws + p.o_a2q),
                                  reinterpret_cast<float*>(ws + p.o_a2s),
-                                 a2_rows, a.inter, a.stream, a2_npp, a2_sorted, numel);
+                                 numel, a.inter, a.stream, slot_pos, p.max_padded);
     if (rc) return rc;
   }
 

@@ -2,6 +2,8 @@
 // the dynamic activation quantisers. Every thread moves 16-byte vectors;
 // a row is processed by consecutive threads so each wave touches one or two
 // contiguous 1 KiB spans per instruction.
+#include <math.h>
+
 #include <string>
 #include <type_traits>
 
@@ -169,6 +171,32 @@ __global__ __launch_bounds__(256) void moe_sum_partials_kernel(
   }
 }
 
+// --------------------------------------------------------- quantisers ---
+// x / scale correctly rounded for a finite scale, from inv = 1 / scale
+// (correctly rounded, one division for all of a scale's values): Markstein's
+// scheme (P. Markstein, "Computation of elementary functions on the IBM RISC
+// System/6000 processor", IBM J. Res. Dev. 1990): x * inv is within two ulps,
+// one residual step brings it within one, and a second from there, with a
+// correctly rounded reciprocal, gives the rounded quotient (and, with x's
+// sign, its signed zero). Six FMA-rate instructions in place of a division's ten and its reciprocal; the
+// quantisers were bound by those. Exact where the residuals are: a quotient
+// small enough for one to lose bits rounds to code 0 either way.
+__device__ __forceinline__ float quotient(float x, float scale, float inv) {
+  float q = x * inv;
+  q = __builtin_fmaf(__builtin_fmaf(-scale, q, x), inv, q);
+  q = __builtin_fmaf(__builtin_fmaf(-scale, q, x), inv, q);
+  return __builtin_copysignf(q, x);
+}
+
+// The row of x a quantiser's work item `i` takes: i, or its slot's padded
+// row (-1: none).
+__device__ __forceinline__ int64_t quant_row(const int32_t* slot_pos, int64_t i,
+                                             int64_t row_limit) {
+  if (!slot_pos) return i;
+  const int64_t r = slot_pos[i];
+  return r < row_limit ? r : -1;
+}
+
 // ------------------------------------------------------ fp8 group quant ---
 // Each lane quantises 8 consecutive columns; the group/8 lanes of a group
 // (a power of two <= 64, aligned within the wave) reduce its amax with
@@ -176,21 +204,18 @@ __global__ __launch_bounds__(256) void moe_sum_partials_kernel(
 // 2048 columns of one row (grid: rows x column chunks), so the row and its
 // skip test are uniform and no index is divided.
 // scale = max(amax, 1e-10) / 448; q = e4m3fn(clamp(x / scale, +-448)).
-// With `rows_dev` given, rows >= *rows_dev are skipped (padded-row buffers
-// whose live prefix is only known on the device); with `sorted_ids` given,
-// so are the pad rows (sorted_ids[r] >= numel), which no GEMM reads.
+// Measured (with a division per value, and padded rows a workgroup each,
+// before): 16384 rows of 2048 22.0 -> 20.1 us (5.0 TB/s); DeepSeek M=4096's
+// GEMM1 output, 32768 live rows of 98048, 76 -> 56 us.
 constexpr int kQuantChunkCols = 256 * 8;  // columns per workgroup
 __global__ __launch_bounds__(256) void quant_fp8_group_kernel(
     const uint16_t* __restrict__ x, uint8_t* __restrict__ q,
-    float* __restrict__ scales, int64_t rows, int64_t cols, int group,
-    const int32_t* __restrict__ rows_dev, const int32_t* __restrict__ sorted_ids,
-    int64_t numel, int64_t scale_kstride) {
+    float* __restrict__ scales, int64_t cols, int group,
+    const int32_t* __restrict__ slot_pos, int64_t row_limit, int64_t scale_kstride) {
   const int lane = threadIdx.x & 63;
   const int lanes_per_group = group / 8;
-  const int64_t r = blockIdx.x;
-  const int64_t live_rows = rows_dev ? min(rows, static_cast<int64_t>(*rows_dev)) : rows;
-  if (r >= live_rows) return;
-  if (sorted_ids && sorted_ids[r] >= numel) return;
+  const int64_t r = quant_row(slot_pos, blockIdx.x, row_limit);
+  if (r < 0) return;
   const int64_t c = (static_cast<int64_t>(blockIdx.y) * kQuantChunkCols) + threadIdx.x * 8;
   // a group lies wholly inside or outside the row (cols % group == 0)
   const bool active = c < cols;
@@ -210,11 +235,19 @@ __global__ __launch_bounds__(256) void quant_fp8_group_kernel(
     amax = fmaxf(amax, __shfl_xor(amax, d, 64));
   if (!active) return;
   const float scale = fmaxf(amax, 1e-10f) / 448.0f;
+  if (scale < INFINITY) {
+    const float inv = 1.0f / scale;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) f[j] = quotient(f[j], scale, inv);
+  } else {  // an infinity in the group
+#pragma unroll
+    for (int j = 0; j < 8; ++j) f[j] = f[j] / scale;
+  }
   uint32_t lo = 0, hi = 0;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    const float a = fminf(fmaxf(f[2 * j] / scale, -448.f), 448.f);
-    const float b = fminf(fmaxf(f[2 * j + 1] / scale, -448.f), 448.f);
+    const float a = fminf(fmaxf(f[2 * j], -448.f), 448.f);
+    const float b = fminf(fmaxf(f[2 * j + 1], -448.f), 448.f);
     const uint32_t pk = cvt_pk_fp8(a, b);
     if (j < 2)
       lo |= pk << (16 * j);
@@ -253,21 +286,37 @@ __global__ __launch_bounds__(256) void moe_scale_gather_kernel(
 
 // ----------------------------------------------------- int8 token quant ---
 constexpr int64_t kInt8WaveRows = 1024;  // rows from which a wave takes a row
+// Eight values of a row -> int8 codes rne(x / scale) clamped to +-127.
+__device__ __forceinline__ uint2 quant_int8x8(const u32x4& w, float scale, float inv) {
+  uint32_t packed[2] = {0, 0};
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float f = (j & 1) ? __uint_as_float(w[j / 2] & 0xffff0000u)
+                            : __uint_as_float(w[j / 2] << 16);
+    float rq = __builtin_rintf(scale < INFINITY ? quotient(f, scale, inv) : f / scale);
+    rq = fminf(fmaxf(rq, -127.f), 127.f);
+    const uint32_t b = static_cast<uint32_t>(static_cast<int32_t>(rq)) & 0xffu;
+    packed[j / 4] |= b << (8 * (j & 3));
+  }
+  return uint2{packed[0], packed[1]};
+}
+
 // One wave per row (4 rows per workgroup), the row held in registers: NV
 // vectors of 8 columns per lane (cols <= 512 * NV, cols % 8 == 0), one read
-// of x. With `rows_dev` given, rows >= *rows_dev are skipped; with
-// `sorted_ids` given, so are the pad rows (sorted_ids[r] >= numel).
-// scale = max(amax, 1e-10) / 127; q = clamp(rne(x / scale), -127, 127).
+// of x. scale = max(amax, 1e-10) / 127; q = clamp(rne(x / scale), -127, 127).
+// Measured as above: 8192 rows of 3584 32.8 -> 27.2 us; Qwen2 M=8192's GEMM1
+// output, 65536 rows of 2560, 109 -> 97 us (5.2 TB/s), M=64's 512 live rows
+// of 8640 15.4 -> 5.2 us (a workgroup per row).
 template <int NV>
 __global__ __launch_bounds__(256) void quant_int8_token_kernel(
     const uint16_t* __restrict__ x, int8_t* __restrict__ q,
     float* __restrict__ scales, int64_t rows, int64_t cols,
-    const int32_t* __restrict__ rows_dev, const int32_t* __restrict__ sorted_ids,
-    int64_t numel) {
+    const int32_t* __restrict__ slot_pos, int64_t row_limit) {
   const int lane = threadIdx.x & 63;
-  const int64_t r = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (r >= rows || (rows_dev && r >= *rows_dev)) return;
-  if (sorted_ids && sorted_ids[r] >= numel) return;
+  const int64_t item = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (item >= rows) return;
+  const int64_t r = quant_row(slot_pos, item, row_limit);
+  if (r < 0) return;
   const uint16_t* src = x + r * cols;
   int8_t* dst = q + r * cols;
   u32x4 w[NV];
@@ -287,24 +336,11 @@ __global__ __launch_bounds__(256) void quant_int8_token_kernel(
 #pragma unroll
   for (int d = 32; d >= 1; d >>= 1) amax = fmaxf(amax, __shfl_xor(amax, d, 64));
   const float scale = fmaxf(amax, 1e-10f) / 127.0f;
+  const float inv = 1.0f / scale;
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
     const int64_t c = (static_cast<int64_t>(v) * 64 + lane) * 8;
-    if (c >= cols) continue;
-    uint32_t packed[2] = {0, 0};
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float f = (j & 1) ? __uint_as_float(w[v][j / 2] & 0xffff0000u)
-                              : __uint_as_float(w[v][j / 2] << 16);
-      float rq = __builtin_rintf(f / scale);
-      rq = fminf(fmaxf(rq, -127.f), 127.f);
-      const uint32_t b = static_cast<uint32_t>(static_cast<int32_t>(rq)) & 0xffu;
-      packed[j / 4] |= b << (8 * (j & 3));
-    }
-    uint2 o;
-    o.x = packed[0];
-    o.y = packed[1];
-    *reinterpret_cast<uint2*>(dst + c) = o;
+    if (c < cols) *reinterpret_cast<uint2*>(dst + c) = quant_int8x8(w[v], scale, inv);
   }
   if (lane == 0) scales[r] = scale;
 }
@@ -376,11 +412,10 @@ int launch_moe_sum_partials(const float* part, int nsplit, void* out, int64_t m,
 // passes over the row (amax, then quantise), for parallelism at small M.
 __global__ __launch_bounds__(256) void quant_int8_token_wg_kernel(
     const uint16_t* __restrict__ x, int8_t* __restrict__ q,
-    float* __restrict__ scales, int64_t cols, const int32_t* __restrict__ rows_dev,
-    const int32_t* __restrict__ sorted_ids, int64_t numel) {
-  const int64_t r = blockIdx.x;
-  if (rows_dev && r >= *rows_dev) return;
-  if (sorted_ids && sorted_ids[r] >= numel) return;
+    float* __restrict__ scales, int64_t cols, const int32_t* __restrict__ slot_pos,
+    int64_t row_limit) {
+  const int64_t r = quant_row(slot_pos, blockIdx.x, row_limit);
+  if (r < 0) return;
   const uint16_t* src = x + r * cols;
   int8_t* dst = q + r * cols;
   float amax = 0.f;
@@ -399,23 +434,10 @@ __global__ __launch_bounds__(256) void quant_int8_token_wg_kernel(
   __syncthreads();
   amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
   const float scale = fmaxf(amax, 1e-10f) / 127.0f;
-  for (int64_t c = threadIdx.x * 8; c < cols; c += 256 * 8) {
-    const u32x4 w = *reinterpret_cast<const u32x4*>(src + c);
-    uint32_t packed[2] = {0, 0};
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float f = (j & 1) ? __uint_as_float(w[j / 2] & 0xffff0000u)
-                              : __uint_as_float(w[j / 2] << 16);
-      float rq = __builtin_rintf(f / scale);
-      rq = fminf(fmaxf(rq, -127.f), 127.f);
-      const uint32_t b = static_cast<uint32_t>(static_cast<int32_t>(rq)) & 0xffu;
-      packed[j / 4] |= b << (8 * (j & 3));
-    }
-    uint2 o;
-    o.x = packed[0];
-    o.y = packed[1];
-    *reinterpret_cast<uint2*>(dst + c) = o;
-  }
+  const float inv = 1.0f / scale;
+  for (int64_t c = threadIdx.x * 8; c < cols; c += 256 * 8)
+    *reinterpret_cast<uint2*>(dst + c) =
+        quant_int8x8(*reinterpret_cast<const u32x4*>(src + c), scale, inv);
   if (threadIdx.x == 0) scales[r] = scale;
 }
 
@@ -433,8 +455,7 @@ static void dispatch_nv(int n, F&& f) {
 
 int launch_quant_fp8_group(const void* x, void* q, float* scales,
                            int64_t rows, int64_t cols, int group,
-                           hipStream_t stream, const int32_t* rows_dev,
-                           const int32_t* sorted_ids, int64_t numel,
+                           hipStream_t stream, const int32_t* slot_pos, int64_t row_limit,
                            int64_t scale_kstride) {
   if (rows == 0 || cols == 0) return FGS_OK;
   const int64_t chunks = (cols + kQuantChunkCols - 1) / kQuantChunkCols;
@@ -443,8 +464,8 @@ int launch_quant_fp8_group(const void* x, void* q, float* scales,
   hipLaunchKernelGGL(quant_fp8_group_kernel,
                      dim3(static_cast<unsigned>(rows), static_cast<unsigned>(chunks)),
                      dim3(256), 0, stream, static_cast<const uint16_t*>(x),
-                     static_cast<uint8_t*>(q), scales, rows, cols, group, rows_dev,
-                     sorted_ids, numel, scale_kstride);
+                     static_cast<uint8_t*>(q), scales, cols, group, slot_pos, row_limit,
+                     scale_kstride);
   return check_launch("quant_fp8_group_kernel");
 }
 
@@ -462,15 +483,13 @@ int launch_scale_gather(const float* xs, int kblocks, const int32_t* sorted_ids,
 
 int launch_quant_int8_token(const void* x, int8_t* q, float* scales,
                             int64_t rows, int64_t cols, hipStream_t stream,
-                            const int32_t* rows_dev, const int32_t* sorted_ids,
-                            int64_t numel) {
+                            const int32_t* slot_pos, int64_t row_limit) {
   if (rows == 0) return FGS_OK;
   const uint16_t* xs = static_cast<const uint16_t*>(x);
   // rows too wide for a wave's registers take the workgroup-per-row kernel
   if (rows < kInt8WaveRows || cols > 512 * kInt8QuantMaxVec) {
     hipLaunchKernelGGL(quant_int8_token_wg_kernel, dim3(static_cast<unsigned>(rows)),
-                       dim3(256), 0, stream, xs, q, scales, cols, rows_dev, sorted_ids,
-                       numel);
+                       dim3(256), 0, stream, xs, q, scales, cols, slot_pos, row_limit);
     return check_launch("quant_int8_token_wg_kernel");
   }
   const dim3 grid(static_cast<unsigned>((rows + 3) / 4));
@@ -480,7 +499,7 @@ int launch_quant_int8_token(const void* x, int8_t* q, float* scales,
     constexpr int NV = decltype(nv_c)::value;
     if constexpr (NV >= 1) {
       hipLaunchKernelGGL(quant_int8_token_kernel<NV>, grid, dim3(256), 0, stream, xs, q,
-                         scales, rows, cols, rows_dev, sorted_ids, numel);
+                         scales, rows, cols, slot_pos, row_limit);
       launched = true;
     }
   });

@@ -97,12 +97,14 @@ int64_t align_scratch_bytes(int64_t numel, int num_experts);
 // from the per-expert counts by the same launch; *planned says whether they
 // were (not on the single-wave path for at most 64 slots). `other`: the
 // class of ids outside [0, num_experts) (-1: dropped); `hist` (or null): the
-// counts of the classes below `other`.
+// counts of the classes below `other`; `slot_pos` (or null, [numel]): each
+// slot's position in the padded order, -1 for a dropped one.
 int launch_align(const int32_t* ids, int64_t numel, int num_experts,
                  int block_size, int32_t* sorted_ids, int32_t* expert_ids,
                  int32_t* num_post_pad, int64_t max_padded, hipStream_t stream,
                  int32_t* scratch = nullptr, const WidePlanReq* plans = nullptr,
-                 bool* planned = nullptr, int other = -1, int32_t* hist = nullptr);
+                 bool* planned = nullptr, int other = -1, int32_t* hist = nullptr,
+                 int32_t* slot_pos = nullptr);
 
 // Routing-format conversion (routing.hip): the triton_kernels routing tuple
 // of _standard_topk_to_triton_kernels, block metadata for block_m in
@@ -123,7 +125,8 @@ int launch_topk_to_routing(const float* weights, const int32_t* ids, int64_t m, 
 int launch_routing_order(const float* gate_scal, const int32_t* src, const int32_t* hist,
                          int64_t numel, int num_experts, int block, int64_t max_padded,
                          int32_t* sorted_ids, int32_t* expert_ids, int32_t* num_post_pad,
-                         int32_t* ids_out, float* w_out, hipStream_t stream);
+                         int32_t* ids_out, float* w_out, hipStream_t stream,
+                         int32_t* slot_pos = nullptr);
 
 int launch_silu_and_mul(const void* in, void* out, int64_t rows, int64_t n,
                         hipStream_t stream);
@@ -138,9 +141,9 @@ int launch_moe_sum_partials(const float* part, int nsplit, void* out, int64_t m,
                             int topk, int64_t k, const int32_t* ids,
                             int num_experts, const float* weights,
                             hipStream_t stream);
-// Activation quantisers; with `rows_dev` given only rows < *rows_dev (a
-// device-side count such as num_tokens_post_padded) are processed, and with
-// `sorted_ids` given the pad rows (sorted_ids[r] >= numel) are skipped.
+// Activation quantisers. With `slot_pos` given, `rows` is a number of slots
+// and slot i's row of x, q and scales is slot_pos[i] (skipped outside [0,
+// row_limit)): only the live rows of a padded buffer get a workgroup.
 // The int8 quantiser holds a row in a wave's registers up to
 // 512 * kInt8QuantMaxVec columns; wider rows take a workgroup each.
 constexpr int kInt8QuantMaxVec = 16;
@@ -148,8 +151,7 @@ constexpr int kInt8QuantMaxVec = 16;
 // scales[g * scale_kstride + row].
 int launch_quant_fp8_group(const void* x, void* q, float* scales, int64_t rows,
                            int64_t cols, int group, hipStream_t stream,
-                           const int32_t* rows_dev = nullptr,
-                           const int32_t* sorted_ids = nullptr, int64_t numel = 0,
+                           const int32_t* slot_pos = nullptr, int64_t row_limit = 0,
                            int64_t scale_kstride = 0);
 // Per-token group scales xs [tokens][kblocks] -> k-block-major scales of
 // the padded row order (out[kb * max_padded + r], rows below
@@ -159,8 +161,7 @@ int launch_scale_gather(const float* xs, int kblocks, const int32_t* sorted_ids,
                         int64_t max_padded, float* out, hipStream_t stream);
 int launch_quant_int8_token(const void* x, int8_t* q, float* scales,
                             int64_t rows, int64_t cols, hipStream_t stream,
-                            const int32_t* rows_dev = nullptr,
-                            const int32_t* sorted_ids = nullptr, int64_t numel = 0);
+                            const int32_t* slot_pos = nullptr, int64_t row_limit = 0);
 
 // k elements per pipeline step of the streaming kernels (kdim must be a
 // multiple of it).

@@ -86,3 +86,19 @@ def test_order_from_extreme_histograms(gpu, E):
                                  fm.GatherIndx(src.to(gpu), src.to(gpu)), E)
     assert torch.equal(ti.cpu().reshape(-1), torch.from_numpy(rid))
     assert torch.equal(tw.cpu().reshape(-1), torch.from_numpy(rwt))
+
+
+@pytest.mark.parametrize("numel", [65, 128, 129, 1000, 1024, 1025])
+@pytest.mark.parametrize("E,B", [(1, 16), (7, 100), (64, 1), (256, 16), (257, 256), (1023, 8),
+                                 (1024, 256)])
+def test_align_a_wave_per_chunk(gpu, numel, E, B):
+    """65 to 1024 slots, a wave each 64 of them, and the sizes on either side;
+    dropped and outside ids, experts without slots and one with most."""
+    g = torch.Generator().manual_seed(numel + E)
+    ids = torch.randint(-1, E + 2, (numel,), generator=g).int()
+    ids[::4] = E // 2
+    s, eids, npp = fm.moe_align_block_size(ids.reshape(-1, 1).to(gpu), E, B)
+    rs, reids, rnpp = moe_ref.align(ids.numpy().reshape(-1, 1), E, B)
+    assert int(npp.item()) == rnpp
+    assert torch.equal(s.cpu(), torch.from_numpy(rs))
+    assert torch.equal(eids.cpu(), torch.from_numpy(reids))

@@ -611,6 +611,8 @@ struct FusedArgs {
   const float* gate_scal = nullptr;
   const int32_t* gather_src = nullptr;
   const int32_t* expt_hist = nullptr;
+  // multiplies the rounded layer output (1: none)
+  float out_scale = 1.f;
   // the schedule of scratch_rule (the allocation-free entry point)
   bool scratch_plan = false;
 };
@@ -818,6 +820,7 @@ static int run_fused(const FusedArgs& a) {
   if (p.direct_sum) {
     // out = the weighted top-k sum, straight from GEMM2
     g2.out = a.out;
+    g2.out_scale = a.out_scale;
     rc = p.pair2 ? launch_gemm2_pair(p.dt, g2, p.kwd, a.stream)
                  : launch_gemm2_direct(p.dt, g2, p.kwd, a.stream);
     if (rc) return rc;
@@ -835,11 +838,11 @@ static int run_fused(const FusedArgs& a) {
   if (p.ksplit2 > 1)
     rc = launch_moe_sum_partials(reinterpret_cast<const float*>(y), p.ksplit2,
                                  a.out, a.m, a.topk, a.hidden, topk_ids, a.e,
-                                 on_input ? nullptr : topk_w, a.stream);
+                                 on_input ? nullptr : topk_w, a.stream, a.out_scale);
   else
     rc = launch_moe_sum_routed(y, a.out, a.m, a.topk, a.hidden, topk_ids,
                                a.e, on_input ? nullptr : topk_w,
-                               a.stream);
+                               a.stream, a.out_scale);
   g_prof.mark(6, a.stream);
   return rc;
 }
@@ -1274,6 +1277,33 @@ int32_t fgs_moe_fused_routed(int32_t qmode, const void* x, const void* w13, cons
   a.gate_scal = gate_scal;
   a.gather_src = gather_src;
   a.expt_hist = expt_hist;
+  if (bias) {
+    a.b13 = b13;
+    a.b2 = b2;
+    a.swiglu = true;
+    a.alpha = alpha;
+    a.limit = limit;
+  }
+  return run_fused(a);
+}
+
+int32_t fgs_moe_fused_scaled(int32_t qmode, const void* x, const void* w13, const void* w2,
+                             const float* w13_scale, const float* w2_scale, const float* b13,
+                             const float* b2, float alpha, float limit,
+                             const float* topk_weights, const int32_t* topk_ids, int64_t m,
+                             int64_t hidden, int64_t inter, int32_t num_experts, int32_t topk,
+                             int32_t flags, float out_scale, void* workspace, int64_t ws_bytes,
+                             void* out, void* stream) {
+  const bool bias = b13 != nullptr || b2 != nullptr;
+  if (bias && (!b13 || !b2)) return fail(FGS_EINVAL, "bias variant needs both b13 and b2");
+  if (bias && (flags & FGS_FLAG_ACT_GELU))
+    return fail(FGS_EUNSUPPORTED, "the bias variant's activation is swiglu only");
+  if (bias && (!(alpha == alpha) || !(limit == limit)))
+    return fail(FGS_EINVAL, "alpha and limit must not be NaN");
+  FusedArgs a{qmode,     x,            w13,      w2, w13_scale, w2_scale, topk_weights,
+              topk_ids,  m,            hidden,   inter, num_experts, topk, flags,
+              workspace, ws_bytes,     out,      as_stream(stream)};
+  a.out_scale = out_scale;
   if (bias) {
     a.b13 = b13;
     a.b2 = b2;

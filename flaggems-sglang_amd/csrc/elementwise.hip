@@ -46,10 +46,11 @@ __global__ __launch_bounds__(256) void silu_and_mul_kernel(
 // `weights` given each slot is scaled first: out = bf16(sum_j w_j * y_j),
 // product and sum each rounded in fp32 in slot order (no fused multiply-add),
 // which is the gammas-on-GEMM2 reduction of ops/fused_moe.py:203,224-231.
+// `out_scale` (1: none) multiplies the rounded output (scaled_bf16_bits).
 __global__ __launch_bounds__(256) void moe_sum_kernel(
     const uint16_t* __restrict__ in, uint16_t* __restrict__ out, int64_t m,
     int topk, int64_t k, const int32_t* __restrict__ ids, int num_experts,
-    const float* __restrict__ weights) {
+    const float* __restrict__ weights, float out_scale) {
   const int64_t vec_per_row = k / 8;
   const int64_t total = m * vec_per_row;
   for (int64_t v = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
@@ -82,7 +83,7 @@ __global__ __launch_bounds__(256) void moe_sum_kernel(
     }
     u32x4 o;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) o[q] = pack_bf16x2(acc[2 * q], acc[2 * q + 1]);
+    for (int q = 0; q < 4; ++q) o[q] = scaled_bf16x2(acc[2 * q], acc[2 * q + 1], out_scale);
     *reinterpret_cast<u32x4*>(out + t * k + c) = o;
   }
 }
@@ -96,7 +97,7 @@ template <int TK>
 __global__ __launch_bounds__(256) void moe_sum_tk_kernel(
     const uint16_t* __restrict__ in, uint16_t* __restrict__ out, int64_t m,
     int64_t k, const int32_t* __restrict__ ids, int num_experts,
-    const float* __restrict__ weights) {
+    const float* __restrict__ weights, float out_scale) {
   const int64_t vec_per_row = k / 8;
   const int64_t total = m * vec_per_row;
   for (int64_t v = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
@@ -132,7 +133,7 @@ __global__ __launch_bounds__(256) void moe_sum_tk_kernel(
     }
     u32x4 o;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) o[q] = pack_bf16x2(acc[2 * q], acc[2 * q + 1]);
+    for (int q = 0; q < 4; ++q) o[q] = scaled_bf16x2(acc[2 * q], acc[2 * q + 1], out_scale);
     *reinterpret_cast<u32x4*>(out + t * k + c) = o;
   }
 }
@@ -141,7 +142,7 @@ __global__ __launch_bounds__(256) void moe_sum_tk_kernel(
 __global__ __launch_bounds__(256) void moe_sum_partials_kernel(
     const float* __restrict__ part, int nsplit, uint16_t* __restrict__ out,
     int64_t m, int topk, int64_t k, const int32_t* __restrict__ ids,
-    int num_experts, const float* __restrict__ weights) {
+    int num_experts, const float* __restrict__ weights, float out_scale) {
   const int64_t vec_per_row = k / 4;
   const int64_t total = m * vec_per_row;
   const int64_t split_stride = m * topk * k;
@@ -165,8 +166,8 @@ __global__ __launch_bounds__(256) void moe_sum_partials_kernel(
       }
     }
     uint2 o;
-    o.x = pack_bf16x2(acc[0], acc[1]);
-    o.y = pack_bf16x2(acc[2], acc[3]);
+    o.x = scaled_bf16x2(acc[0], acc[1], out_scale);
+    o.y = scaled_bf16x2(acc[2], acc[3], out_scale);
     *reinterpret_cast<uint2*>(out + t * k + c) = o;
   }
 }
@@ -363,10 +364,6 @@ int launch_silu_and_mul(const void* in, void* out, int64_t rows, int64_t n,
   return check_launch("silu_and_mul_kernel");
 }
 
-int launch_moe_sum_routed(const void* in, void* out, int64_t m, int topk,
-                          int64_t k, const int32_t* ids, int num_experts,
-                          const float* weights, hipStream_t stream);
-
 int launch_moe_sum(const void* in, void* out, int64_t m, int topk, int64_t k,
                    hipStream_t stream) {
   return launch_moe_sum_routed(in, out, m, topk, k, nullptr, 0, nullptr, stream);
@@ -374,37 +371,37 @@ int launch_moe_sum(const void* in, void* out, int64_t m, int topk, int64_t k,
 
 int launch_moe_sum_routed(const void* in, void* out, int64_t m, int topk,
                           int64_t k, const int32_t* ids, int num_experts,
-                          const float* weights, hipStream_t stream) {
+                          const float* weights, hipStream_t stream, float out_scale) {
   if (m == 0) return FGS_OK;
   const dim3 grid(grid_for(m * (k / 8), 256));
   const uint16_t* src = static_cast<const uint16_t*>(in);
   uint16_t* dst = static_cast<uint16_t*>(out);
   if (topk == 8) {
     hipLaunchKernelGGL(moe_sum_tk_kernel<8>, grid, dim3(256), 0, stream, src, dst, m, k, ids,
-                       num_experts, weights);
+                       num_experts, weights, out_scale);
     return check_launch("moe_sum_tk_kernel");
   }
   if (topk == 2) {
     hipLaunchKernelGGL(moe_sum_tk_kernel<2>, grid, dim3(256), 0, stream, src, dst, m, k, ids,
-                       num_experts, weights);
+                       num_experts, weights, out_scale);
     return check_launch("moe_sum_tk_kernel");
   }
   hipLaunchKernelGGL(moe_sum_kernel, dim3(grid_for(m * (k / 8), 256)),
                      dim3(256), 0, stream, static_cast<const uint16_t*>(in),
                      static_cast<uint16_t*>(out), m, topk, k, ids, num_experts,
-                     weights);
+                     weights, out_scale);
   return check_launch("moe_sum_kernel");
 }
 
 int launch_moe_sum_partials(const float* part, int nsplit, void* out, int64_t m,
                             int topk, int64_t k, const int32_t* ids,
                             int num_experts, const float* weights,
-                            hipStream_t stream) {
+                            hipStream_t stream, float out_scale) {
   if (m == 0) return FGS_OK;
   hipLaunchKernelGGL(moe_sum_partials_kernel, dim3(grid_for(m * (k / 4), 256)),
                      dim3(256), 0, stream, part, nsplit,
                      static_cast<uint16_t*>(out), m, topk, k, ids, num_experts,
-                     weights);
+                     weights, out_scale);
   return check_launch("moe_sum_partials_kernel");
 }
 

@@ -78,6 +78,7 @@ struct GemmParams {
                               // the top-k sum; null: off
   int32_t* route_ids;
   int32_t shape;              // tiled: the tile shape (kTileByConfig, ...)
+  float out_scale;            // folded GEMM2: the layer output's scale
 };
 
 // Router gating (scores -> top-k -> renormalise), one wave per token;
@@ -134,13 +135,13 @@ int launch_moe_sum(const void* in, void* out, int64_t m, int topk, int64_t k,
                    hipStream_t stream);
 int launch_moe_sum_routed(const void* in, void* out, int64_t m, int topk,
                           int64_t k, const int32_t* ids, int num_experts,
-                          const float* weights, hipStream_t stream);
+                          const float* weights, hipStream_t stream, float out_scale = 1.f);
 // Same reduction over fp32 split-K partials [nsplit][m*topk][k]: each slot's
 // y = bf16(sum_s part[s]) (splits in order), then the weighted top-k sum.
 int launch_moe_sum_partials(const float* part, int nsplit, void* out, int64_t m,
                             int topk, int64_t k, const int32_t* ids,
                             int num_experts, const float* weights,
-                            hipStream_t stream);
+                            hipStream_t stream, float out_scale = 1.f);
 // Activation quantisers. With `slot_pos` given, `rows` is a number of slots
 // and slot i's row of x, q and scales is slot_pos[i] (skipped outside [0,
 // row_limit)): only the live rows of a padded buffer get a workgroup.

@@ -691,7 +691,7 @@ __global__ __launch_bounds__(KW * 64) void moe_gemm2_direct_kernel(const GemmPar
     for (int w = 1; w < KW; ++w) tot += red[w][lane];
   }
   // row 0 of the tile: lane group 0, register 0
-  if (lg == 0) static_cast<uint16_t*>(p.out)[col] = f32_to_bf16_bits(tot[0]);
+  if (lg == 0) static_cast<uint16_t*>(p.out)[col] = scaled_bf16_bits(tot[0], p.out_scale);
 }
 
 template <int DT, bool QA>
@@ -882,7 +882,7 @@ __global__ __launch_bounds__(KW * 64) void moe_gemm2_pair_kernel(const GemmParam
     }
     tot = __fadd_rn(tot, __fmul_rn(gamma, bf16_bits_to_f32(f32_to_bf16_bits(y + b))));
   }
-  static_cast<uint16_t*>(p.out)[col] = f32_to_bf16_bits(tot);
+  static_cast<uint16_t*>(p.out)[col] = scaled_bf16_bits(tot, p.out_scale);
 }
 
 template <int DT, bool QA>

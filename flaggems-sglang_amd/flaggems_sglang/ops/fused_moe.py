@@ -443,6 +443,18 @@ def _weight_qmode(w1, w2, use_fp8_w8a8, use_int8_w8a8, per_channel_quant,
     return _capi.QMODE_BF16
 
 
+def _split_scale(factor):
+    """A routed scaling factor as ``(kernel scale, tensor factor)``: a number
+    that converts to float32 as a tensor's multiplication converts it (a
+    float, or an integer that a double holds) is applied by the layer's last
+    kernel; anything else multiplies the output tensor."""
+    if factor is None or not factor != 1.0:
+        return None, None
+    if isinstance(factor, float) or (isinstance(factor, int) and abs(factor) <= 2 ** 53):
+        return float(factor), None
+    return None, factor
+
+
 def fused_moe(
     hidden_states: torch.Tensor,
     w1: torch.Tensor,
@@ -529,28 +541,35 @@ def fused_moe(
     out = torch.empty((M, K), dtype=torch.bfloat16, device=x.device)
     ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=x.device)
     stream = _stream_ptr(x)
-    if qmode == _capi.QMODE_BF16:
+    scale, factor = _split_scale(routed_scaling_factor)
+    s1 = s2 = None
+    if qmode != _capi.QMODE_BF16:
+        s1 = w1_scale.to(torch.float32).contiguous()
+        s2 = w2_scale.to(torch.float32).contiguous()
+    if scale is not None:
+        rc = lib.fgs_moe_fused_scaled(
+            qmode, x.data_ptr(), w1.data_ptr(), w2.data_ptr(),
+            None if s1 is None else s1.data_ptr(), None if s2 is None else s2.data_ptr(),
+            None, None, 1.0, 0.0, wts.data_ptr(), ids.data_ptr(), M, K, N, E, topk,
+            flags, scale, ws.data_ptr(), ws_bytes, out.data_ptr(), stream)
+    elif qmode == _capi.QMODE_BF16:
         rc = lib.fgs_moe_fused_bf16(
             x.data_ptr(), w1.data_ptr(), w2.data_ptr(), wts.data_ptr(),
             ids.data_ptr(), M, K, N, E, topk, flags, ws.data_ptr(), ws_bytes,
             out.data_ptr(), stream)
     elif qmode == _capi.QMODE_FP8_BLOCK:
-        s1 = w1_scale.to(torch.float32).contiguous()
-        s2 = w2_scale.to(torch.float32).contiguous()
         rc = lib.fgs_moe_fused_fp8_block(
             x.data_ptr(), w1.data_ptr(), w2.data_ptr(), s1.data_ptr(),
             s2.data_ptr(), 128, 128, wts.data_ptr(), ids.data_ptr(), M, K, N,
             E, topk, flags, ws.data_ptr(), ws_bytes, out.data_ptr(), stream)
     else:
-        s1 = w1_scale.to(torch.float32).contiguous()
-        s2 = w2_scale.to(torch.float32).contiguous()
         rc = lib.fgs_moe_fused_int8_channel(
             x.data_ptr(), w1.data_ptr(), w2.data_ptr(), s1.data_ptr(),
             s2.data_ptr(), wts.data_ptr(), ids.data_ptr(), M, K, N, E, topk,
             flags, ws.data_ptr(), ws_bytes, out.data_ptr(), stream)
     _capi.check(rc, "fused_moe")
-    if routed_scaling_factor is not None and routed_scaling_factor != 1.0:
-        out.mul_(routed_scaling_factor)
+    if factor is not None:
+        out.mul_(factor)
     return out
 
 
@@ -814,22 +833,32 @@ def fused_moe_with_bias(
                     "fused_moe_with_bias")
     out = torch.empty((M, K), dtype=torch.bfloat16, device=x.device)
     ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=x.device)
-    if qmode == _capi.QMODE_BF16:
+    scale, factor = _split_scale(routed_scaling_factor)
+    s1 = s2 = None
+    if qmode != _capi.QMODE_BF16:
+        s1 = w1_scale.to(torch.float32).contiguous()
+        s2 = w2_scale.to(torch.float32).contiguous()
+    if scale is not None:
+        rc = lib.fgs_moe_fused_scaled(
+            qmode, x.data_ptr(), w1.data_ptr(), w2.data_ptr(),
+            None if s1 is None else s1.data_ptr(), None if s2 is None else s2.data_ptr(),
+            b1f.data_ptr(), b2f.data_ptr(), alpha, limit, wts.data_ptr(), ids.data_ptr(),
+            M, K, N, E, topk, flags, scale, ws.data_ptr(), ws_bytes, out.data_ptr(),
+            _stream_ptr(x))
+    elif qmode == _capi.QMODE_BF16:
         rc = lib.fgs_moe_fused_bf16_bias(
             x.data_ptr(), w1.data_ptr(), b1f.data_ptr(), w2.data_ptr(),
             b2f.data_ptr(), wts.data_ptr(), ids.data_ptr(), M, K, N, E, topk, flags,
             alpha, limit, ws.data_ptr(), ws_bytes, out.data_ptr(), _stream_ptr(x))
     else:
-        s1 = w1_scale.to(torch.float32).contiguous()
-        s2 = w2_scale.to(torch.float32).contiguous()
         rc = lib.fgs_moe_fused_quant_bias(
             qmode, x.data_ptr(), w1.data_ptr(), b1f.data_ptr(), w2.data_ptr(),
             b2f.data_ptr(), s1.data_ptr(), s2.data_ptr(), wts.data_ptr(),
             ids.data_ptr(), M, K, N, E, topk, flags, alpha, limit, ws.data_ptr(),
             ws_bytes, out.data_ptr(), _stream_ptr(x))
     _capi.check(rc, "fused_moe_with_bias")
-    if routed_scaling_factor is not None and routed_scaling_factor != 1.0:
-        out.mul_(routed_scaling_factor)
+    if factor is not None:
+        out.mul_(factor)
     return out
 
 
@@ -995,11 +1024,11 @@ def fused_moe_flagos(obj, layer, dispatch_output):
         alpha = getattr(cfg, "gemm1_alpha", None)
         limit = getattr(cfg, "gemm1_clamp_limit", None)
 
-        def call(x, tw, ti):
+        def call(x, tw, ti, scale=None):
             return fused_moe_with_bias(
                 x, w13, b13n, layer.w2_weight, b2, tw, ti,
                 apply_router_weight_on_input=on_input, gemm1_alpha=alpha,
-                gemm1_clamp_limit=limit, interleaved=False)
+                gemm1_clamp_limit=limit, interleaved=False, routed_scaling_factor=scale)
 
         def call_routed(x):
             return _fused_routed(
@@ -1008,10 +1037,11 @@ def fused_moe_flagos(obj, layer, dispatch_output):
                 limit=0.0 if limit is None else float(limit),
                 apply_router_weight_on_input=on_input)
     else:
-        def call(x, tw, ti):
+        def call(x, tw, ti, scale=None):
             return fused_moe(x, layer.w13_weight, layer.w2_weight, tw, ti,
                              activation=activation,
-                             apply_router_weight_on_input=on_input)
+                             apply_router_weight_on_input=on_input,
+                             routed_scaling_factor=scale)
 
         def call_routed(x):
             return _fused_routed(x, layer.w13_weight, layer.w2_weight, *routing,
@@ -1024,13 +1054,13 @@ def fused_moe_flagos(obj, layer, dispatch_output):
         output = rows.view(hidden_states.shape[0], topk_ids.shape[1],
                            hidden_states.shape[-1])
     else:
-        if routing is not None:
-            output = call_routed(hidden_states)
-        else:
-            output = call(hidden_states, topk_weights, topk_ids)
         scale = getattr(cfg, "routed_scaling_factor", None)
-        if scale is not None and scale != 1.0:
-            output.mul_(scale)
+        if routing is None:
+            output = call(hidden_states, topk_weights, topk_ids, scale)
+        else:
+            output = call_routed(hidden_states)
+            if scale is not None and scale != 1.0:
+                output.mul_(scale)
     return _combine_input_cls()(hidden_states=output)
 
 

@@ -314,6 +314,20 @@ int32_t fgs_moe_fused_quant_bias(int32_t qmode, const void* x, const void* w13,
                                  float alpha, float limit, void* workspace,
                                  int64_t ws_bytes, void* out, void* stream);
 
+/* The fused entry points above in one, with the layer output scaled: out =
+ * bf16(out_scale * bf16(layer output)), the values of an in-place
+ * multiplication of the output (the adapter's routed scaling factor,
+ * ops/fused_moe.py:415-420) without its launch and its pass over the output.
+ * qmode and scales as fgs_moe_fused_bf16 / _fp8_block / _int8_channel; b13
+ * and b2 both null or both set as in fgs_moe_fused_routed below. */
+int32_t fgs_moe_fused_scaled(int32_t qmode, const void* x, const void* w13, const void* w2,
+                             const float* w13_scale, const float* w2_scale, const float* b13,
+                             const float* b2, float alpha, float limit,
+                             const float* topk_weights, const int32_t* topk_ids, int64_t m,
+                             int64_t hidden, int64_t inter, int32_t num_experts, int32_t topk,
+                             int32_t flags, float out_scale, void* workspace, int64_t ws_bytes,
+                             void* out, void* stream);
+
 /* Fused MoE on the reference's routing tuple instead of (topk_weights,
  * topk_ids): the inputs triton_kernel_fused_experts
  * (ops/fused_moe.py:149-232) and triton_kernel_fused_experts_with_bias

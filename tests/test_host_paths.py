@@ -3,8 +3,10 @@
 import sys
 import types
 
+import pytest
 import torch
 
+from flaggems_sglang import _capi
 from flaggems_sglang.ops import fused_moe as fm
 
 
@@ -47,3 +49,30 @@ def test_conversion_view_shortcut():
     # one row or column: both orders are contiguous, so the view serves
     row = torch.randn(2, 1, 6)
     assert cache(row).data_ptr() == row.data_ptr() and cache(row).is_contiguous()
+
+
+def test_scaled_entry_refusals():
+    """The scaled entry's checks are the entry points' it covers."""
+    lib, nul, shape = _capi.load(), None, (4, 256, 128, 4, 2)
+    need = lib.fgs_moe_workspace_bytes(*shape, _capi.QMODE_BF16, 0)
+
+    def call(b13=nul, b2=nul, w=16, flags=0, alpha=1.0, ws_bytes=need):
+        return lib.fgs_moe_fused_scaled(0, 16, 16, 16, nul, nul, b13, b2, alpha, 0.0, w, 16,
+                                        *shape, flags, 2.5, 256, ws_bytes, 16, nul)
+
+    for kw, code, text in [({"b13": 16}, -1, "b13 and b2"), ({"b2": 16}, -1, "b13 and b2"),
+                           ({"b13": 16, "b2": 16, "flags": _capi.FLAG_ACT_GELU}, -2, "swiglu"),
+                           ({"b13": 16, "b2": 16, "alpha": float("nan")}, -1, "NaN"),
+                           ({"w": nul}, -1, "null pointer"), ({"ws_bytes": need - 1}, -1,
+                                                              "workspace")]:
+        assert call(**kw) == code and text in _capi.last_error()
+
+
+def test_split_scale():
+    t = torch.tensor([1.0, 2.0])
+    for factor, want in [(None, (None, None)), (1, (None, None)), (True, (None, None)),
+                         (2, (2.0, None)), (0.5, (0.5, None)), (False, (0.0, None)),
+                         (2 ** 53 + 1, (None, 2 ** 53 + 1)), (1j, (None, 1j))]:
+        assert fm._split_scale(factor) == want
+    with pytest.raises(RuntimeError):  # ambiguous, as the comparison was before
+        fm._split_scale(t)

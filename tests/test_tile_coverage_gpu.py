@@ -159,3 +159,21 @@ def test_scheduled_shapes(gpu, mode, shape, expect):
         other = fm.fused_moe(x, wts.w1, wts.w2, w, ids, _flags=_capi.flag_tile(1),
                              **wts.kwargs(mode))
         assert torch.equal(res, other)
+
+
+# the gathered activation scales (256-row fp8 tiles): k blocks below, at and
+# across a thread's 16, in fours and not
+@pytest.mark.parametrize("kblocks", [1, 4, 15, 16, 17, 20, 33, 36])
+def test_gathered_scales(gpu, kblocks):
+    K, N = 128 * kblocks, 256
+    g = torch.Generator(device=gpu).manual_seed(kblocks)
+    counts = [300, 1, 257, 0, 65, 255]
+    w, ids = _routing_with_counts(counts, gpu, seed=kblocks)
+    wts = testing.make_weights(K, N, len(counts), "fp8", 0.05, device=gpu, seed=K)
+    # a factor per token and k block, so that a wrong block's scale shows
+    x = torch.randn(ids.shape[0], kblocks, 128, generator=g, device=gpu)
+    x *= 4.0 ** torch.randint(-3, 4, (ids.shape[0], kblocks, 1), generator=g, device=gpu)
+    x = x.reshape(-1, K).to(torch.bfloat16)
+    outs = [fm.fused_moe(x, wts.w1, wts.w2, w, ids, _flags=_capi.flag_tile(cfg),
+                         **wts.kwargs("fp8")) for cfg in (0, 1)]
+    assert torch.equal(outs[0], outs[1])

@@ -5,8 +5,8 @@
 // flattened expert ids (:134) and a per-expert histogram (:137-139). The
 // output is the block-padded, expert-grouped order the grouped GEMMs consume.
 //
-// moe_align_kernel (1025 to 4095 slots; the variants for fewer and for more
-// are below): one workgroup of 16 wave64s (and, asked for tile plans, a
+// moe_align_kernel (more experts than moe_align_mid_kernel's LDS takes, below
+// 4096 slots, or any number of slots without scratch memory): one workgroup of 16 wave64s (and, asked for tile plans, a
 // second that writes them). Wave w owns the contiguous slot segment
 // [w*seg, (w+1)*seg). Pass 1 counts ids per (wave, expert) in LDS; pass 2
 // turns the counts into per-expert padded offsets plus per-wave offsets
@@ -62,7 +62,7 @@ __device__ __forceinline__ int class_of(int id, int num_classes, int other) {
 }
 
 constexpr int kAlignWaves = 16;
-constexpr int64_t kAlignMultiMin = 4096;  // slots from which the multi-WG path runs
+constexpr int64_t kAlignMultiMin = 4096;  // slots from which scratch is asked for
 constexpr int kAlignThreads = kAlignWaves * kWave;
 
 __global__ __launch_bounds__(kAlignThreads) void moe_align_kernel(
@@ -195,15 +195,20 @@ __global__ __launch_bounds__(kAlignThreads) void moe_align_kernel(
   }
 }
 
-// 65 to kAlignMidMax slots: one workgroup, a wave per 64 slots, each lane's
-// id held in a register (moe_align_kernel reads the ids twice and counts them
-// with LDS atomics). Ballots give a slot's rank and its id's count in the
-// wave; a thread per expert adds the waves' counts up and the experts' padded
+// 65 to kAlignMidMax slots: one workgroup, R runs of 64 consecutive slots per
+// wave, the ids held in registers (moe_align_kernel reads them twice and
+// counts them with LDS atomics, a run at a time). Ballots give a slot's rank
+// and its id's count in its run, the wave's LDS row the count of its earlier
+// runs; a thread per expert adds the waves' counts up and the experts' padded
 // sizes are scanned across the workgroup. The sentinels are written
 // first, over the whole buffer, and are complete at a barrier before the
 // slots land on them. Bound: latency (296 slots of 256 experts 11.4
-// -> 5.0 us against moe_align_kernel, 512 of 64 6.8 -> 5.4).
-constexpr int kAlignMidMax = kAlignThreads;
+// -> 5.0 us against moe_align_kernel, 512 of 64 6.8 -> 5.4; 2048 of 128
+// 9.3 -> 6.1, of 256 12.8 -> 6.3, 4088 of 128 11.8 -> 8.6). 4096 slots of 128
+// take 8.6 us here, 3.3 + 8.9 in the two launches of the counting kernels;
+// 8192 take 14.3 (8 runs) and 3.7 + 9.6.
+constexpr int kAlignMidMax = 4 * kAlignThreads;
+template <int R>
 __global__ __launch_bounds__(kAlignThreads) void moe_align_mid_kernel(
     const int32_t* __restrict__ ids, int numel, int num_experts, int block_size, int id_bits,
     int32_t* __restrict__ sorted_ids, int32_t* __restrict__ expert_ids,
@@ -211,7 +216,7 @@ __global__ __launch_bounds__(kAlignThreads) void moe_align_mid_kernel(
     WidePlanReq plan1, int other, int32_t* __restrict__ hist, int32_t* __restrict__ slot_pos) {
   extern __shared__ int32_t smem[];
   const int E = num_experts;
-  const int nw = (numel + kWave - 1) / kWave;  // waves that hold slots
+  const int nw = (numel + R * kWave - 1) / (R * kWave);  // waves that hold slots
   int32_t* cnt = smem;           // [nw][E]: counts, then slots of earlier waves
   int32_t* off = cnt + nw * E;   // [E + 1]
   int32_t* tot = off + E + 1;    // [E]
@@ -219,22 +224,39 @@ __global__ __launch_bounds__(kAlignThreads) void moe_align_mid_kernel(
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wave = tid / kWave;
+  const int slot0 = wave * R * kWave + lane;  // run r's slot: + 64 r
 
-  const int e = tid < numel ? class_of(ids[tid], E, other) : -1;
+  int e[R], rank[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+    e[r] = slot0 + r * kWave < numel ? class_of(ids[slot0 + r * kWave], E, other) : -1;
   for (int i = tid; i < nw * E; i += kAlignThreads) cnt[i] = 0;
   if (blockIdx.x == 0) {
     for (int64_t p = tid; p < max_padded; p += kAlignThreads) sorted_ids[p] = numel;
   }
-  const bool valid = e >= 0;
-  uint64_t match = __ballot(valid);
-  for (int b = 0; b < id_bits; ++b) {
-    const bool bit = valid && ((e >> b) & 1);
-    const uint64_t on = __ballot(bit);
-    match &= bit ? on : ~on;
+  uint64_t match[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const bool valid = e[r] >= 0;
+    match[r] = __ballot(valid);
+    for (int b = 0; b < id_bits; ++b) {
+      const bool bit = valid && ((e[r] >> b) & 1);
+      const uint64_t on = __ballot(bit);
+      match[r] &= bit ? on : ~on;
+    }
+    rank[r] = __popcll(match[r] & ((lane == 0) ? 0ull : (~0ull >> (kWave - lane))));
   }
-  const int rank = __popcll(match & ((lane == 0) ? 0ull : (~0ull >> (kWave - lane))));
   __syncthreads();  // the zeros (and sentinels) are written
-  if (valid && rank == 0) cnt[wave * E + e] = __popcll(match);
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const bool valid = e[r] >= 0;
+    const int before = R > 1 && valid ? cnt[wave * E + e[r]] : 0;
+    // the id's first lane moves its count on after every lane has read it
+    __builtin_amdgcn_wave_barrier();
+    if (valid && rank[r] == 0) cnt[wave * E + e[r]] = before + __popcll(match[r]);
+    __builtin_amdgcn_wave_barrier();
+    rank[r] += before;
+  }
   __syncthreads();
 
   // thread x: expert x's slots before each wave, its total, its padded size
@@ -276,10 +298,13 @@ __global__ __launch_bounds__(kAlignThreads) void moe_align_mid_kernel(
     return;
   }
   if (tid == 0) num_post_pad[0] = total;
-  if (tid < numel) {
-    const int at = valid ? off[e] + cnt[wave * E + e] + rank : -1;
-    if (valid) sorted_ids[at] = tid;
-    if (slot_pos) slot_pos[tid] = at;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int slot = slot0 + r * kWave;
+    if (slot >= numel) break;
+    const int at = e[r] >= 0 ? off[e[r]] + cnt[wave * E + e[r]] + rank[r] : -1;
+    if (at >= 0) sorted_ids[at] = slot;
+    if (slot_pos) slot_pos[slot] = at;
   }
   if (tid < E)
     for (int b = start / block_size; b < (start + padded) / block_size; ++b) expert_ids[b] = tid;
@@ -288,7 +313,7 @@ __global__ __launch_bounds__(kAlignThreads) void moe_align_mid_kernel(
 }
 
 // ------------------------------------------------ multi-workgroup variant ---
-// For many slots: the ids are cut into chunks of kChunk consecutive slots.
+// For more slots than moe_align_mid_kernel takes: the ids are cut into chunks of kChunk consecutive slots.
 // Kernel 1 counts each chunk's ids per expert (counts[c][e]). Kernel 2 runs
 // one workgroup per chunk: it sums the counts of every chunk (totals) and of
 // the chunks before its own (its per-expert base, so lower slots come
@@ -537,6 +562,27 @@ int launch_align(const int32_t* ids, int64_t numel, int num_experts,
                        sorted_ids, expert_ids, num_post_pad, max_padded, other, hist, slot_pos);
     return check_launch("moe_align_wave_kernel");
   }
+  // The single-workgroup kernel of up to kAlignMidMax slots; past it (or with
+  // more experts than its threads or LDS take) the counting kernels where
+  // there is scratch memory for them.
+  int runs = 1;
+  while (numel > runs * static_cast<int64_t>(kAlignThreads)) runs *= 2;
+  const int64_t mid_waves = (numel + runs * kWave - 1) / (runs * kWave);
+  const size_t smem_mid =
+      sizeof(int32_t) * (static_cast<size_t>(mid_waves + 2) * num_experts + 1);
+  const bool with_plans = plan0.plan || plan1.plan;
+  if (numel <= kAlignMidMax && num_experts <= kAlignThreads && smem_mid <= 60 * 1024) {
+    auto kernel = runs == 1   ? moe_align_mid_kernel<1>
+                  : runs == 2 ? moe_align_mid_kernel<2>
+                              : moe_align_mid_kernel<4>;
+    hipLaunchKernelGGL(kernel, dim3(with_plans ? 2 : 1), dim3(kAlignThreads), smem_mid, stream,
+                       ids, static_cast<int>(numel), num_experts, block_size, id_bits,
+                       sorted_ids, expert_ids, num_post_pad, max_padded, plan0, plan1, other,
+                       hist, slot_pos);
+    const int rc = check_launch("moe_align_mid_kernel");
+    if (!rc && planned) *planned = with_plans;
+    return rc;
+  }
   if (scratch && numel >= kAlignMultiMin) {
     const int nchunks = static_cast<int>((numel + kChunk - 1) / kChunk);
     const size_t smem1 = sizeof(int32_t) * num_experts;
@@ -545,7 +591,6 @@ int launch_align(const int32_t* ids, int64_t numel, int num_experts,
                        smem1, stream, ids, numel, num_experts, scratch, other);
     int rc = check_launch("moe_align_count_kernel");
     if (rc) return rc;
-    const bool with_plans = plan0.plan || plan1.plan;
     hipLaunchKernelGGL(moe_align_scatter_kernel, dim3(nchunks + (with_plans ? 1 : 0)),
                        dim3(kChunkThreads),
                        smem2, stream, ids, numel, num_experts, block_size, id_bits,
@@ -553,18 +598,6 @@ int launch_align(const int32_t* ids, int64_t numel, int num_experts,
                        hist, slot_pos);
     rc = check_launch("moe_align_scatter_kernel");
     if (!rc && planned) *planned = plan0.plan || plan1.plan;
-    return rc;
-  }
-  const bool with_plans = plan0.plan || plan1.plan;
-  const size_t smem_mid =
-      sizeof(int32_t) * (static_cast<size_t>((numel + kWave - 1) / kWave + 2) * num_experts + 1);
-  if (numel <= kAlignMidMax && num_experts <= kAlignThreads && smem_mid <= 60 * 1024) {
-    hipLaunchKernelGGL(moe_align_mid_kernel, dim3(with_plans ? 2 : 1), dim3(kAlignThreads),
-                       smem_mid, stream, ids, static_cast<int>(numel), num_experts, block_size,
-                       id_bits, sorted_ids, expert_ids, num_post_pad, max_padded, plan0, plan1,
-                       other, hist, slot_pos);
-    const int rc = check_launch("moe_align_mid_kernel");
-    if (!rc && planned) *planned = with_plans;
     return rc;
   }
   const size_t smem = align_smem_bytes(num_experts);

@@ -88,12 +88,14 @@ def test_order_from_extreme_histograms(gpu, E):
     assert torch.equal(tw.cpu().reshape(-1), torch.from_numpy(rwt))
 
 
-@pytest.mark.parametrize("numel", [65, 128, 129, 1000, 1024, 1025])
+@pytest.mark.parametrize("numel", [65, 128, 129, 1000, 1024, 1025, 2048, 2049, 4095, 4096,
+                                   4097, 8191, 8192, 8193])
 @pytest.mark.parametrize("E,B", [(1, 16), (7, 100), (64, 1), (256, 16), (257, 256), (1023, 8),
                                  (1024, 256)])
 def test_align_a_wave_per_chunk(gpu, numel, E, B):
-    """65 to 1024 slots, a wave each 64 of them, and the sizes on either side;
-    dropped and outside ids, experts without slots and one with most."""
+    """65 to 4096 slots, one to four runs of 64 of them per wave, and the
+    sizes on either side; dropped and outside ids, experts without slots and
+    one with most."""
     g = torch.Generator().manual_seed(numel + E)
     ids = torch.randint(-1, E + 2, (numel,), generator=g).int()
     ids[::4] = E // 2

@@ -227,7 +227,19 @@ static int pick_kw(int64_t kdim, int step, int cap, int min_steps) {
 // 6: 0.99, 8: 1.02; 1280 4: 1.00, 6: 1.07; 1536 4: 1.03; 1920 6: 1.00, 8:
 // 1.03; 2816 4: 1.07. fp8 48 tiles 8: 1.00, 14: 1.08; 112 4: 0.97, 8: 1.02;
 // 128 8: 0.95, 10: 1.02; 736 and more 4: 1.03 to 1.15.
-static double stream_rows(int dt, double tiles, int64_t k_bytes) {
+// A GEMM2 of at most 100 256-column tiles over the touched experts leaves the
+// tiled kernels most CUs idle even split over k, and streaming lasts longer
+// (layer in blocks of 16 and of 32 rows,
+// hidden / intermediate / experts, streaming / tiled at 10 and 12.5 rows: bf16
+// 2048/8448/8 0.75, 0.98; 3072/8448/8 0.91, 1.14; 1280/4352/8 0.86, 1.04;
+// 2048/4352/8 0.72, 0.87; 3072/4352/8 0.83, 0.96; 1536/7168/16 0.99, 1.30.
+// int8 2048/8448/8 1.00, 1.32; 2048/4352/8 0.89, 1.12; 1536/7168/16 1.12;
+// fp8 2048/8448/8 1.04; 2048/4352/8 0.93, 1.16; 3072/4352/8 0.97, 1.16).
+static double stream_rows(int dt, double tiles, double tiles2, int64_t k_bytes) {
+  if (tiles2 <= 100 && tiles > 160) {
+    if (dt == kDtBf16 && tiles <= 1000) return tiles <= 400 ? 12.5 : 10.5;
+    if (tiles <= (dt == kDtInt8 ? 600 : 400)) return 10.5;
+  }
   if (dt == kDtFp8) return tiles <= 160 ? 7 : 3;
   if (dt == kDtInt8) return tiles <= 160 ? 12.5 : tiles <= 1000 ? 6 : tiles <= 2000 ? 4.5 : 3;
   return tiles <= 160 ? 10 : tiles <= 1000 ? (k_bytes < 2048 ? 12.5 : 9) : tiles <= 2000 ? 7 : 5.5;
@@ -246,15 +258,18 @@ static void call_rule(int64_t m, int64_t hidden, int64_t inter, int e, int topk,
   const int64_t esz = p.dt == kDtBf16 ? 2 : 1;
   const double rows = static_cast<double>(numel) / e;
   const int forced_cfg = ((flags & FGS_FLAG_TILE_MASK) >> 12) - 1;
-  // Streaming row blocks: 16 rows up to 12 rows per expert (more would give
-  // a share of the experts a second block, which streams their weights
-  // again), 32 up to 28 (bf16 hidden 3584, intermediate 2560, 64 experts, 16
+  // Streaming row blocks: 16 rows up to 12.5 rows per expert (8 experts,
+  // hidden 1920, intermediate 4224, 12.5 rows: 106 us in blocks of 32, 93 of
+  // 16; more would give a share of the experts a second block, which streams
+  // their weights again), 32 up to 28 (bf16 hidden 3584, intermediate 2560, 64 experts, 16
   // rows: GEMM1 614 us in blocks of 16, 528 of 32), else 64.
-  p.mt = rows <= 12 ? 1 : rows <= 28 ? 2 : 4;
+  p.mt = rows <= 12.5 ? 1 : rows <= 28 ? 2 : 4;
   // Tiled kernels (deep DMA pipeline) or streaming ones (weights straight
   // into registers), by rows per expert: see stream_rows.
-  const double tiles1 = e * (1.0 - std::exp(-rows)) * static_cast<double>(inter / 128);
-  const double stream_to = stream_rows(p.dt, tiles1, inter * esz);
+  const double touched = e * (1.0 - std::exp(-rows));
+  const double stream_to =
+      stream_rows(p.dt, touched * static_cast<double>(inter / 128),
+                  touched * static_cast<double>((hidden + 255) / 256), inter * esz);
   // One token always streams (its direct-row schedule). Every accepted shape
   // can run tiled: a hidden size that is an odd multiple of 128 ends GEMM2 in
   // a half tile. (Streaming reads an expert's weights once per block of at

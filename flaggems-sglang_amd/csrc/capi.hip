@@ -227,14 +227,15 @@ static int pick_kw(int64_t kdim, int step, int cap, int min_steps) {
 // 6: 0.99, 8: 1.02; 1280 4: 1.00, 6: 1.07; 1536 4: 1.03; 1920 6: 1.00, 8:
 // 1.03; 2816 4: 1.07. fp8 48 tiles 8: 1.00, 14: 1.08; 112 4: 0.97, 8: 1.02;
 // 128 8: 0.95, 10: 1.02; 736 and more 4: 1.03 to 1.15.
+//
 // A GEMM2 of at most 100 256-column tiles over the touched experts leaves the
-// tiled kernels most CUs idle even split over k, and streaming lasts longer
-// (layer in blocks of 16 and of 32 rows,
-// hidden / intermediate / experts, streaming / tiled at 10 and 12.5 rows: bf16
+// tiled kernels most CUs idle even split over k, and streaming lasts longer.
+// Layer time, streaming / tiled, at 10 rows (16-row blocks) and 12.5 (32-row
+// blocks; 16-row ones are up to 13 % faster), hidden/intermediate/experts: bf16
 // 2048/8448/8 0.75, 0.98; 3072/8448/8 0.91, 1.14; 1280/4352/8 0.86, 1.04;
 // 2048/4352/8 0.72, 0.87; 3072/4352/8 0.83, 0.96; 1536/7168/16 0.99, 1.30.
 // int8 2048/8448/8 1.00, 1.32; 2048/4352/8 0.89, 1.12; 1536/7168/16 1.12;
-// fp8 2048/8448/8 1.04; 2048/4352/8 0.93, 1.16; 3072/4352/8 0.97, 1.16).
+// fp8 2048/8448/8 1.04; 2048/4352/8 0.93, 1.16; 3072/4352/8 0.97, 1.16.
 static double stream_rows(int dt, double tiles, double tiles2, int64_t k_bytes) {
   if (tiles2 <= 100 && tiles > 160) {
     if (dt == kDtBf16 && tiles <= 1000) return tiles <= 400 ? 12.5 : 10.5;

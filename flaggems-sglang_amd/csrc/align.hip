@@ -303,11 +303,14 @@ __global__ __launch_bounds__(kAlignThreads) void moe_align_mid_kernel(
     const int slot = slot0 + r * kWave;
     if (slot >= numel) break;
     const int at = e[r] >= 0 ? off[e[r]] + cnt[wave * E + e[r]] + rank[r] : -1;
-    if (at >= 0) sorted_ids[at] = slot;
     if (slot_pos) slot_pos[slot] = at;
+    if (at < 0) continue;
+    sorted_ids[at] = slot;
+    // a block's first row names its expert: every slot at once (one thread
+    // walking its expert's blocks took 80 us more for 3584 blocks of one row)
+    const uint32_t b = static_cast<uint32_t>(at) / static_cast<uint32_t>(block_size);
+    if (b * block_size == static_cast<uint32_t>(at)) expert_ids[b] = e[r];
   }
-  if (tid < E)
-    for (int b = start / block_size; b < (start + padded) / block_size; ++b) expert_ids[b] = tid;
   for (int64_t b = total / block_size + tid; b < max_padded / block_size; b += kAlignThreads)
     expert_ids[b] = -1;
 }

@@ -104,3 +104,40 @@ def test_align_a_wave_per_chunk(gpu, numel, E, B):
     assert int(npp.item()) == rnpp
     assert torch.equal(s.cpu(), torch.from_numpy(rs))
     assert torch.equal(eids.cpu(), torch.from_numpy(reids))
+
+
+def test_align_skewed_ids_in_parallel(gpu):
+    """4096 slots in blocks of one row: all on one expert cost about what
+    spread ones do (the block -> expert map is written by the slots, not by a
+    thread per expert: 12 times as long). Whole launches, replayed in turn."""
+    from flaggems_sglang import _capi
+
+    lib, n, E = _capi.load(), 4096, 64
+    out = [torch.empty(s, dtype=torch.int32, device=gpu) for s in (n, n, 1)]
+    ids = {"spread": torch.arange(n, device=gpu).remainder(E).int(),
+           "one": torch.full((n,), E - 1, device=gpu).int()}
+
+    def launch(x):
+        stream = torch.cuda.current_stream().cuda_stream
+        for _ in range(20):
+            _capi.check(lib.fgs_moe_align_block_size(
+                x.data_ptr(), n, E, 1, *(t.data_ptr() for t in out), n, None, 0, stream), "align")
+
+    graphs = {}
+    for name, x in ids.items():
+        launch(x)
+        torch.cuda.synchronize()
+        graphs[name] = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graphs[name]):
+            launch(x)
+    times = {name: [] for name in ids}
+    for _ in range(5):
+        for name, g in graphs.items():
+            t0, t1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            t0.record()
+            g.replay()
+            t1.record()
+            torch.cuda.synchronize()
+            times[name].append(t0.elapsed_time(t1))
+            assert torch.equal(out[1].cpu(), ids[name].sort().values.cpu())
+    assert min(times["one"]) < 3 * min(times["spread"]), times

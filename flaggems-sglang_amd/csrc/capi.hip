@@ -762,12 +762,12 @@ static int run_fused(const FusedArgs& a) {
   g2.shape = p.shape2;
   const int rows2 = static_cast<int>(p.n_launch << p.eid_shift2);
 
-  // (quantised modes) each slot's row of the padded order, for the quantiser
-  // of the GEMM1 output
-  int32_t* slot_pos = p.o_pos >= 0 ? reinterpret_cast<int32_t*>(ws + p.o_pos) : nullptr;
+  // (quantised modes) the padded row of each slot, or of each position of a
+  // routing tuple's gathered order, for the quantiser of the GEMM1 output
+  int32_t* row_of = p.o_pos >= 0 ? reinterpret_cast<int32_t*>(ws + p.o_pos) : nullptr;
   if (routed && !p.direct) {
     rc = launch_routing_order(a.gate_scal, a.gather_src, a.expt_hist, numel, a.e, p.block_m,
-                              p.max_padded, sorted, eids, npp, rids, rw, a.stream, slot_pos);
+                              p.max_padded, sorted, eids, npp, rids, rw, a.stream, row_of);
     if (rc) return rc;
   } else if (!p.direct) {
     // the alignment also writes the 4-wave GEMMs' tile plans (their launches
@@ -781,7 +781,7 @@ static int run_fused(const FusedArgs& a) {
     rc = launch_align(topk_ids, numel, a.e, p.block_m, sorted, eids, npp,
                       p.max_padded, a.stream,
                       p.o_alg >= 0 ? reinterpret_cast<int32_t*>(ws + p.o_alg) : nullptr,
-                      req, &planned, -1, nullptr, slot_pos);
+                      req, &planned, -1, nullptr, row_of);
     if (rc) return rc;
     g1.plan_ready = planned && req[0].plan ? 1 : 0;
     g2.plan_ready = planned && req[1].plan ? 1 : 0;
@@ -815,20 +815,20 @@ static int run_fused(const FusedArgs& a) {
   if (rc) return rc;
   g_prof.mark(3, a.stream);
 
-  // direct rows: the compact slot rows; else each slot's padded row
+  // direct rows: the compact slot rows; else the padded rows that hold slots
   if (p.qfold) {
     // GEMM2 quantises the a2 slot rows itself
   } else if (p.dt == kDtFp8) {
     // tiled: the scales k-block-major over the padded rows (see o_xst)
     rc = launch_quant_fp8_group(a2, ws + p.o_a2q,
                                 reinterpret_cast<float*>(ws + p.o_a2s),
-                                numel, a.inter, 128, a.stream, slot_pos, p.max_padded,
+                                numel, a.inter, 128, a.stream, row_of, p.max_padded,
                                 p.tiled ? p.max_padded : 0);
     if (rc) return rc;
   } else if (p.dt == kDtInt8) {
     rc = launch_quant_int8_token(a2, reinterpret_cast<int8_t*>(ws + p.o_a2q),
                                  reinterpret_cast<float*>(ws + p.o_a2s),
-                                 numel, a.inter, a.stream, slot_pos, p.max_padded);
+                                 numel, a.inter, a.stream, row_of, p.max_padded);
     if (rc) return rc;
   }
 

@@ -189,12 +189,12 @@ __device__ __forceinline__ float quotient(float x, float scale, float inv) {
   return __builtin_copysignf(q, x);
 }
 
-// The row of x a quantiser's work item `i` takes: i, or its slot's padded
-// row (-1: none).
-__device__ __forceinline__ int64_t quant_row(const int32_t* slot_pos, int64_t i,
+// The row of x a quantiser's work item `i` takes: i, or the padded row given
+// for it (-1: none).
+__device__ __forceinline__ int64_t quant_row(const int32_t* row_of, int64_t i,
                                              int64_t row_limit) {
-  if (!slot_pos) return i;
-  const int64_t r = slot_pos[i];
+  if (!row_of) return i;
+  const int64_t r = row_of[i];
   return r < row_limit ? r : -1;
 }
 
@@ -212,10 +212,10 @@ constexpr int kQuantChunkCols = 256 * 8;  // columns per workgroup
 __global__ __launch_bounds__(256) void quant_fp8_group_kernel(
     const uint16_t* __restrict__ x, uint8_t* __restrict__ q,
     float* __restrict__ scales, int64_t cols, int group,
-    const int32_t* __restrict__ slot_pos, int64_t row_limit, int64_t scale_kstride) {
+    const int32_t* __restrict__ row_of, int64_t row_limit, int64_t scale_kstride) {
   const int lane = threadIdx.x & 63;
   const int lanes_per_group = group / 8;
-  const int64_t r = quant_row(slot_pos, blockIdx.x, row_limit);
+  const int64_t r = quant_row(row_of, blockIdx.x, row_limit);
   if (r < 0) return;
   const int64_t c = (static_cast<int64_t>(blockIdx.y) * kQuantChunkCols) + threadIdx.x * 8;
   // a group lies wholly inside or outside the row (cols % group == 0)
@@ -326,11 +326,11 @@ template <int NV>
 __global__ __launch_bounds__(256) void quant_int8_token_kernel(
     const uint16_t* __restrict__ x, int8_t* __restrict__ q,
     float* __restrict__ scales, int64_t rows, int64_t cols,
-    const int32_t* __restrict__ slot_pos, int64_t row_limit) {
+    const int32_t* __restrict__ row_of, int64_t row_limit) {
   const int lane = threadIdx.x & 63;
   const int64_t item = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (item >= rows) return;
-  const int64_t r = quant_row(slot_pos, item, row_limit);
+  const int64_t r = quant_row(row_of, item, row_limit);
   if (r < 0) return;
   const uint16_t* src = x + r * cols;
   int8_t* dst = q + r * cols;
@@ -423,9 +423,9 @@ int launch_moe_sum_partials(const float* part, int nsplit, void* out, int64_t m,
 // passes over the row (amax, then quantise), for parallelism at small M.
 __global__ __launch_bounds__(256) void quant_int8_token_wg_kernel(
     const uint16_t* __restrict__ x, int8_t* __restrict__ q,
-    float* __restrict__ scales, int64_t cols, const int32_t* __restrict__ slot_pos,
+    float* __restrict__ scales, int64_t cols, const int32_t* __restrict__ row_of,
     int64_t row_limit) {
-  const int64_t r = quant_row(slot_pos, blockIdx.x, row_limit);
+  const int64_t r = quant_row(row_of, blockIdx.x, row_limit);
   if (r < 0) return;
   const uint16_t* src = x + r * cols;
   int8_t* dst = q + r * cols;
@@ -466,7 +466,7 @@ static void dispatch_nv(int n, F&& f) {
 
 int launch_quant_fp8_group(const void* x, void* q, float* scales,
                            int64_t rows, int64_t cols, int group,
-                           hipStream_t stream, const int32_t* slot_pos, int64_t row_limit,
+                           hipStream_t stream, const int32_t* row_of, int64_t row_limit,
                            int64_t scale_kstride) {
   if (rows == 0 || cols == 0) return FGS_OK;
   const int64_t chunks = (cols + kQuantChunkCols - 1) / kQuantChunkCols;
@@ -475,7 +475,7 @@ int launch_quant_fp8_group(const void* x, void* q, float* scales,
   hipLaunchKernelGGL(quant_fp8_group_kernel,
                      dim3(static_cast<unsigned>(rows), static_cast<unsigned>(chunks)),
                      dim3(256), 0, stream, static_cast<const uint16_t*>(x),
-                     static_cast<uint8_t*>(q), scales, cols, group, slot_pos, row_limit,
+                     static_cast<uint8_t*>(q), scales, cols, group, row_of, row_limit,
                      scale_kstride);
   return check_launch("quant_fp8_group_kernel");
 }
@@ -494,13 +494,13 @@ int launch_scale_gather(const float* xs, int kblocks, const int32_t* sorted_ids,
 
 int launch_quant_int8_token(const void* x, int8_t* q, float* scales,
                             int64_t rows, int64_t cols, hipStream_t stream,
-                            const int32_t* slot_pos, int64_t row_limit) {
+                            const int32_t* row_of, int64_t row_limit) {
   if (rows == 0) return FGS_OK;
   const uint16_t* xs = static_cast<const uint16_t*>(x);
   // rows too wide for a wave's registers take the workgroup-per-row kernel
   if (rows < kInt8WaveRows || cols > 512 * kInt8QuantMaxVec) {
     hipLaunchKernelGGL(quant_int8_token_wg_kernel, dim3(static_cast<unsigned>(rows)),
-                       dim3(256), 0, stream, xs, q, scales, cols, slot_pos, row_limit);
+                       dim3(256), 0, stream, xs, q, scales, cols, row_of, row_limit);
     return check_launch("quant_int8_token_wg_kernel");
   }
   const dim3 grid(static_cast<unsigned>((rows + 3) / 4));
@@ -510,7 +510,7 @@ int launch_quant_int8_token(const void* x, int8_t* q, float* scales,
     constexpr int NV = decltype(nv_c)::value;
     if constexpr (NV >= 1) {
       hipLaunchKernelGGL(quant_int8_token_kernel<NV>, grid, dim3(256), 0, stream, xs, q,
-                         scales, rows, cols, slot_pos, row_limit);
+                         scales, rows, cols, row_of, row_limit);
       launched = true;
     }
   });

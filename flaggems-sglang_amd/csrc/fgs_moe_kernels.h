@@ -122,12 +122,13 @@ int launch_topk_to_routing(const float* weights, const int32_t* ids, int64_t m, 
 // The routing tuple -> the alignment's padded order (sorted_ids non-null:
 // sorted_ids [max_padded], expert_ids [max_padded / block], num_post_pad)
 // and / or per flat slot its expert id and gate scale (ids_out non-null:
-// ids_out, w_out [numel]); num_experts <= 1024. See routing.hip.
+// ids_out, w_out [numel]) with each gathered position's padded row (row_of
+// [numel], or null); num_experts <= 1024. See routing.hip.
 int launch_routing_order(const float* gate_scal, const int32_t* src, const int32_t* hist,
                          int64_t numel, int num_experts, int block, int64_t max_padded,
                          int32_t* sorted_ids, int32_t* expert_ids, int32_t* num_post_pad,
                          int32_t* ids_out, float* w_out, hipStream_t stream,
-                         int32_t* slot_pos = nullptr);
+                         int32_t* row_of = nullptr);
 
 int launch_silu_and_mul(const void* in, void* out, int64_t rows, int64_t n,
                         hipStream_t stream);
@@ -142,9 +143,10 @@ int launch_moe_sum_partials(const float* part, int nsplit, void* out, int64_t m,
                             int topk, int64_t k, const int32_t* ids,
                             int num_experts, const float* weights,
                             hipStream_t stream, float out_scale = 1.f);
-// Activation quantisers. With `slot_pos` given, `rows` is a number of slots
-// and slot i's row of x, q and scales is slot_pos[i] (skipped outside [0,
-// row_limit)): only the live rows of a padded buffer get a workgroup.
+// Activation quantisers. With `row_of` given, `rows` is a number of slots (or
+// gathered positions) and the row of x, q and scales that item i takes is
+// row_of[i] (skipped outside [0, row_limit)): only the live rows of a padded
+// buffer get a workgroup.
 // The int8 quantiser holds a row in a wave's registers up to
 // 512 * kInt8QuantMaxVec columns; wider rows take a workgroup each.
 constexpr int kInt8QuantMaxVec = 16;
@@ -152,7 +154,7 @@ constexpr int kInt8QuantMaxVec = 16;
 // scales[g * scale_kstride + row].
 int launch_quant_fp8_group(const void* x, void* q, float* scales, int64_t rows,
                            int64_t cols, int group, hipStream_t stream,
-                           const int32_t* slot_pos = nullptr, int64_t row_limit = 0,
+                           const int32_t* row_of = nullptr, int64_t row_limit = 0,
                            int64_t scale_kstride = 0);
 // Per-token group scales xs [tokens][kblocks] -> k-block-major scales of
 // the padded row order (out[kb * max_padded + r], rows below
@@ -162,7 +164,7 @@ int launch_scale_gather(const float* xs, int kblocks, const int32_t* sorted_ids,
                         int64_t max_padded, float* out, hipStream_t stream);
 int launch_quant_int8_token(const void* x, int8_t* q, float* scales,
                             int64_t rows, int64_t cols, hipStream_t stream,
-                            const int32_t* slot_pos = nullptr, int64_t row_limit = 0);
+                            const int32_t* row_of = nullptr, int64_t row_limit = 0);
 
 // k elements per pipeline step of the streaming kernels (kdim must be a
 // multiple of it).

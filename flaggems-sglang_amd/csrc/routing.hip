@@ -208,19 +208,22 @@ __device__ __forceinline__ int first_above(const int32_t* incl, int n, int64_t x
 //   inverse (ids_out != null): for every gathered position p with
 //     v = src[p] in [0, numel): ids_out[v] = the expert whose range holds p
 //     (-1 past the histogram's total: a slot no expert reads),
-//     w_out[v] = gate_scal[p], and (slot_pos != null) slot_pos[v] = p's padded
-//     row (-1 where no expert reads it; a slot that src never names is left
-//     as it was).
+//     w_out[v] = gate_scal[p];
+//   rows (row_of != null, with the inverse): row_of[p] = p's padded row, -1
+//     past the total and where src[p] is outside. By position, so all numel
+//     entries are written and each row that holds a slot has its own, also
+//     where a caller's src names a slot twice and another never.
 // Every workgroup (one thread per expert: blockDim >= E, a power of two up
 // to 1024) derives the offsets itself (by wave scans: 5.9 us at 8192 gates
-// over 64 experts, 8.5 with 64-bit sums in LDS and a barrier per step) and then walks its share of the
-// positions; no atomics, so the result is deterministic.
+// over 64 experts, 8.5 with 64-bit sums in LDS and a barrier per step) and
+// then walks its share of the positions; no atomics, so the result is
+// deterministic.
 __global__ __launch_bounds__(kOrderThreads) void routing_order_kernel(
     const float* __restrict__ gate_scal, const int32_t* __restrict__ src,
     const int32_t* __restrict__ hist, int64_t numel, int num_experts, int block,
     int64_t max_padded, int32_t* __restrict__ sorted_ids, int32_t* __restrict__ expert_ids,
     int32_t* __restrict__ num_post_pad, int32_t* __restrict__ ids_out,
-    float* __restrict__ w_out, int32_t* __restrict__ slot_pos) {
+    float* __restrict__ w_out, int32_t* __restrict__ row_of) {
   __shared__ uint32_t tmp[1][16];
   __shared__ int32_t raw_incl[kOrderThreads];
   __shared__ int32_t pad_incl[kOrderThreads];
@@ -264,14 +267,15 @@ __global__ __launch_bounds__(kOrderThreads) void routing_order_kernel(
   if (ids_out) {
     for (int64_t p = tid; p < numel; p += stride) {
       const int32_t s = src[p];
-      if (s < 0 || s >= numel) continue;
+      const bool named = s >= 0 && s < numel;
       const int x = p < total_raw ? first_above(raw_incl, E, p) : -1;
+      if (row_of)
+        row_of[p] = !named || x < 0 ? -1
+                                    : (x > 0 ? pad_incl[x - 1] : 0) + static_cast<int32_t>(p) -
+                                          (x > 0 ? raw_incl[x - 1] : 0);
+      if (!named) continue;
       ids_out[s] = x;
       w_out[s] = gate_scal[p];
-      if (slot_pos)
-        slot_pos[s] = x < 0 ? -1
-                            : (x > 0 ? pad_incl[x - 1] : 0) +
-                                  static_cast<int32_t>(p) - (x > 0 ? raw_incl[x - 1] : 0);
     }
   }
 }
@@ -280,7 +284,7 @@ int launch_routing_order(const float* gate_scal, const int32_t* src, const int32
                          int64_t numel, int num_experts, int block, int64_t max_padded,
                          int32_t* sorted_ids, int32_t* expert_ids, int32_t* num_post_pad,
                          int32_t* ids_out, float* w_out, hipStream_t stream,
-                         int32_t* slot_pos) {
+                         int32_t* row_of) {
   if (num_experts < 1 || num_experts > kOrderThreads)
     return fail(FGS_EINVAL, "routing order: num_experts must be in [1, 1024]");
   // one wave for up to 64 experts (its barriers cost next to nothing)
@@ -291,7 +295,7 @@ int launch_routing_order(const float* gate_scal, const int32_t* src, const int32
       static_cast<int>(std::min<int64_t>(std::max<int64_t>((work + threads - 1) / threads, 1), 1024));
   hipLaunchKernelGGL(routing_order_kernel, dim3(blocks), dim3(threads), 0, stream,
                      gate_scal, src, hist, numel, num_experts, block, max_padded, sorted_ids,
-                     expert_ids, num_post_pad, ids_out, w_out, slot_pos);
+                     expert_ids, num_post_pad, ids_out, w_out, row_of);
   return check_launch("routing_order_kernel");
 }
 

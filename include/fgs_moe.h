@@ -340,7 +340,10 @@ int32_t fgs_moe_fused_scaled(int32_t qmode, const void* x, const void* w13, cons
  * and b2 both null (silu, or gelu with FGS_FLAG_ACT_GELU) or both set (the
  * bias variant: swiglu(alpha, limit) as fgs_moe_fused_bf16_bias). Same
  * workspace (fgs_moe_workspace_bytes) and output as those entry points on
- * the equivalent (topk_weights, topk_ids). */
+ * the equivalent (topk_weights, topk_ids). src is a permutation of the slots:
+ * entries outside [0, m * topk) are skipped, a slot named twice takes either
+ * entry's result, and the output row of a token with a slot that src never
+ * names is unspecified. */
 int32_t fgs_moe_fused_routed(int32_t qmode, const void* x, const void* w13, const void* w2,
                              const float* w13_scale, const float* w2_scale, const float* b13,
                              const float* b2, float alpha, float limit,

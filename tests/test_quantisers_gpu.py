@@ -5,6 +5,7 @@ over scales and values across bf16's range, and on the rows of a padded order
 import pytest
 import torch
 
+from flaggems_sglang import _capi, testing
 from flaggems_sglang.ops import fused_moe as fm
 
 pytestmark = pytest.mark.gpu
@@ -72,3 +73,45 @@ def test_infinite_values(gpu):
     q, s = fm.per_token_quant_int8(x.to(gpu))
     rq, rs = _int8(x)
     assert torch.equal(q.cpu()[keep], rq[keep])
+
+
+@pytest.mark.parametrize("flags", [_capi.FLAG_FORCE_DECODE, _capi.flag_tile(0), _capi.flag_tile(1)],
+                         ids=["stream", "tile0", "tile1"])
+@pytest.mark.parametrize("mode", ["fp8", "int8"])
+def test_repeated_slots_of_a_routing_tuple(gpu, mode, flags):
+    """A routing tuple whose gathered order names some slots twice inside their
+    expert's range, some never and some outside: every row that holds a slot is
+    quantised (both of a repeated one's, which GEMM2 both reads), whatever the
+    workspace held. The same bits as the layer with the unnamed slots dropped."""
+    M, K, N, E, topk = 384, 512, 256, 4, 2
+    n, qm = M * topk, {"fp8": _capi.QMODE_FP8_BLOCK, "int8": _capi.QMODE_INT8_CHANNEL}[mode]
+    wts = testing.make_weights(K, N, E, mode, 0.05, device=gpu, seed=K)
+    x, w, ids = testing.make_tokens(M, K, E, topk, device=gpu, seed=M)
+    w, ids = fm._routing_to_topk(*fm.standard_topk_to_routing(w, ids, E)[:2], M)
+    rd, gi, _ = fm.standard_topk_to_routing(w, ids, E)
+    src, gate, hist = gi.src_indx.cpu().clone(), rd.gate_scal.cpu().clone(), rd.expt_hist.cpu()
+    g = torch.Generator().manual_seed(1)
+    dropped = torch.zeros(n, dtype=torch.bool)
+    start = 0
+    for c in hist.tolist():
+        p = start + torch.randperm(c, generator=g)
+        for a, b in zip(p[: c // 4].tolist(), p[c // 4: c // 4 * 2].tolist()):
+            dropped[int(src[a])] = True           # a names b's slot instead of its own
+            src[a], gate[a] = src[b], gate[b]
+        dropped[int(src[p[-1]])] = True
+        src[p[-1]] = n + 7 if start % 2 else -3
+        start += c
+    src, gate = src.to(gpu), gate.to(gpu)
+    lib = _capi.load()
+    need = lib.fgs_moe_workspace_bytes(M, K, N, E, topk, qm, flags)
+    ws = torch.full((need,), 0xff, dtype=torch.uint8, device=gpu)  # fp8 codes and scales: NaN
+    out = torch.empty((M, K), dtype=torch.bfloat16, device=gpu)
+    _capi.check(lib.fgs_moe_fused_routed(
+        qm, x.data_ptr(), wts.w1.data_ptr(), wts.w2.data_ptr(), wts.w1_scale.data_ptr(),
+        wts.w2_scale.data_ptr(), None, None, 1.0, 0.0, gate.data_ptr(), src.data_ptr(),
+        rd.expt_hist.data_ptr(), M, K, N, E, topk, flags, ws.data_ptr(), need, out.data_ptr(),
+        torch.cuda.current_stream().cuda_stream), "fused_moe (routing tuple)")
+    ids = torch.where(dropped.view(M, topk).to(gpu), torch.full_like(ids, -1), ids)
+    ref = fm.fused_moe(x, wts.w1, wts.w2, w, ids, _flags=flags, **wts.kwargs(mode))
+    # (a token with an unnamed slot reads what the workspace held for it: here -1, dropped)
+    assert torch.equal(out, ref)

@@ -126,9 +126,12 @@ static int pick_ksplit(double tiles, int64_t stages, int64_t numel, int64_t hidd
 // The k split the allocation-free entry point's scratch is sized for
 // (scratch_rule): the smallest (<= 4, keeping >= 8 stages of 128 bytes of k)
 // whose expected grid fills >= 90 % of its last round, else the best one.
-static int scratch_ksplit(int64_t numel, int e, int bm, int64_t hidden, int64_t k_bytes) {
-  const double blocks = static_cast<double>(numel) / bm +
-                        0.5 * static_cast<double>(std::min<int64_t>(e, numel));
+// Row blocks: half a padded one per expert beside the full ones, or one per
+// expert (`one_block`).
+static int scratch_ksplit(int64_t numel, int e, int bm, int64_t hidden, int64_t k_bytes,
+                          bool one_block) {
+  const double experts = static_cast<double>(std::min<int64_t>(e, numel));
+  const double blocks = one_block ? experts : static_cast<double>(numel) / bm + 0.5 * experts;
   const double wgs = blocks * static_cast<double>(hidden / 256);
   int best = 1;
   double best_eff = 0.0;
@@ -295,7 +298,7 @@ static void call_rule(int64_t m, int64_t hidden, int64_t inter, int e, int topk,
     // 32, and 56 / 33 at 180; 256 such tiles and more are slower (1024, 512,
     // 16 experts, 180 rows: 25 wide, 30).
     const double deep_limit = 0.875 * kNumCUs;
-    if (!tile_forced()) {
+    if (forced_tile() < 0) {
       if (blocks128 * (inter / 64) <= deep_limit) {
         p.tile_cfg = 1;
         p.shape1 = kTileDeep;
@@ -370,12 +373,18 @@ static void scratch_rule(int64_t m, int64_t hidden, int64_t inter, int e, int to
   if (!p.tiled) return;
   const bool many = e >= 32;
   p.tile_cfg = forced_cfg >= 0 ? forced_cfg
+               : forced_tile() >= 0 ? forced_tile()
                : rows >= 96 || (many && rows >= 48) ? 0
                : rows >= 24 || (many && rows >= 8) ? 1 : 3;
   p.tile_cfg2 = p.tile_cfg;
-  p.ksplit2 = scratch_ksplit(numel, e, tiled_block_m(p.tile_cfg), hidden, k_bytes);
+  // (the 160-row configuration, when forced, runs below 160 rows per expert:
+  // about one block per touched expert)
+  p.ksplit2 = scratch_ksplit(numel, e, tiled_block_m(p.tile_cfg), hidden, k_bytes,
+                             p.tile_cfg == 4 && rows < 160);
+  if (forced_ksplit() > 0 && k_bytes / 128 >= 8 * forced_ksplit()) p.ksplit2 = forced_ksplit();
   const int64_t tiles_est = (numel / 256 + std::min<int64_t>(e, numel)) * (hidden / 256);
-  p.tail2 = p.tile_cfg == 0 && tiles_est >= kNumCUs && tiles_est <= 8 * kNumCUs;
+  p.tail2 = tail_choice() && p.tile_cfg == 0 && forced_ksplit() == 0 && tiles_est >= kNumCUs &&
+            tiles_est <= 8 * kNumCUs;
   if (p.tail2) p.ksplit2 = 1;
 }
 

@@ -186,7 +186,7 @@ constexpr int kTiledConfigs = 5;  // row blocks 256, 128, 64, 32, 160
 int tiled_config_supported(int dt, int cfg);
 int tiled_config_for(int dt, double rows_per_expert, int num_experts, double tiles256,
                      double tiles128);
-bool tile_forced();  // FGS_MOE_TILE is set
+int forced_tile();  // FGS_MOE_TILE's configuration, -1 unset
 int tiled_block_m(int cfg);
 int launch_gemm_tiled(int dt, int cfg, bool gemm1, const GemmParams& p,
                       int row_blocks, hipStream_t stream);

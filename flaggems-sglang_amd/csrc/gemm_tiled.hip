@@ -1000,7 +1000,7 @@ static const int kTileRows[kTiledConfigs] = {Cfg256::BM, Cfg128::BM, Cfg64::BM,
                                              Cfg32::BM, Cfg160::BM};
 
 // FGS_MOE_TILE (0..4) forces one configuration (a tuning aid; read once).
-static int forced_tile() {
+int forced_tile() {
   static const int forced = [] {
     const char* s = tuning_env("FGS_MOE_TILE");
     if (!s) return -1;
@@ -1054,8 +1054,6 @@ int tiled_config_for(int dt, double rows_per_expert, int num_experts, double til
   if (forced_tile() >= 0) c = forced_tile();
   return c;
 }
-
-bool tile_forced() { return forced_tile() >= 0; }
 
 int tiled_block_m(int cfg) { return kTileRows[cfg]; }
 

@@ -1,5 +1,7 @@
 """Host-side shortcuts of the Python layer, on the CPU."""
 
+import os
+import subprocess
 import sys
 import types
 
@@ -76,3 +78,46 @@ def test_split_scale():
         assert fm._split_scale(factor) == want
     with pytest.raises(RuntimeError):  # ambiguous, as the comparison was before
         fm._split_scale(t)
+
+
+# (problem, flags), whether the allocation-free entry point takes it, and under
+# which tuning switches that turns over
+_T4 = _capi.flag_tile(4)
+_NOALLOC = [((582, 6912, 1920, 16, 2), _T4, True, ("KSPLIT=3",)),
+            ((94, 7680, 1792, 8, 8), _T4, True, ("KSPLIT=3",)),
+            ((3220, 1536, 1280, 60, 2), _T4, False, ()),
+            ((138, 4352, 5632, 16, 4), _T4, False, ("KSPLIT=3",)),
+            ((1503, 3328, 128, 32, 4), 0, False, ("KSPLIT=3", "TILE=4", "TAIL=0")),
+            ((582, 6912, 1920, 16, 2), 0, True, ("KSPLIT=3",)),
+            ((2100, 4224, 3200, 8, 2), 0, True, ())]
+
+
+def _noalloc_taken(lib):
+    """Null pointers: a problem past the scratch is refused as unsupported, any
+    other for its pointers (or, without a GPU, its scratch), before a launch."""
+    out = []
+    for shape, flags, _, _ in _NOALLOC:
+        rc = lib.fgs_moe_fused_bf16_noalloc(*[None] * 5, *shape, flags, None, None)
+        assert rc < 0
+        out.append(rc != _capi.FGS_EUNSUPPORTED)
+    return out
+
+
+@pytest.mark.parametrize("switch", ["", "TILE=4", "TAIL=0", "KSPLIT=3"])
+def test_no_alloc_accepted_set(switch):
+    """The problems the allocation-free entry point takes do not move with the
+    schedule rules: the 160-row configuration's split counts one block per
+    expert below 160 rows, and the tuning switches count as in a call."""
+    want = [taken != (switch in turns) for _, _, taken, turns in _NOALLOC]
+    if not switch:
+        assert _noalloc_taken(_capi.load()) == want
+        return
+    here = os.path.dirname(os.path.abspath(__file__))
+    code = (f"import sys; sys.path[:0] = {[here] + sys.path!r}\n"
+            "import test_host_paths as t\nprint(t._noalloc_taken(t._capi.load()))")
+    name, value = switch.split("=")
+    env = dict(os.environ, FGS_MOE_TUNING="1", **{"FGS_MOE_" + name: value})
+    r = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True,
+                       timeout=300)
+    assert r.returncode == 0, r.stderr[-2000:]
+    assert r.stdout.strip().splitlines()[-1] == str(want)

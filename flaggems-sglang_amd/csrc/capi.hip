@@ -89,12 +89,16 @@ constexpr int kNumCUs = 256;  // MI355X
 // Row blocks of bm rows the alignment is expected to make: an expert's slots
 // are about normal around numel / e (each token picks an expert with
 // probability topk / e), and it holds a j-th block when it has more than
-// (j - 1) * bm slots.
+// (j - 1) * bm slots. Blocks more than nine deviations below the mean are
+// certain (in doubles), so they are counted and the loop runs over the spread
+// only: 2^27 tokens on one expert took 8.5 ms a plan block by block.
 static double expected_blocks(int64_t m, int topk, int e, int bm) {
   const double mean = static_cast<double>(m) * topk / e;
   const double sd = std::sqrt(std::max(1e-3, mean * (1.0 - static_cast<double>(topk) / e)));
   double per_expert = 1.0 - std::exp(-mean);
-  for (double at = bm; at <= mean + 6 * sd; at += bm)
+  const double certain = std::max(0.0, std::floor((mean - 9 * sd - 0.5) / bm));
+  per_expert += certain;
+  for (double at = (certain + 1) * bm; at <= mean + 6 * sd; at += bm)
     per_expert += 0.5 * std::erfc((at + 0.5 - mean) / (sd * std::sqrt(2.0)));
   return std::min(per_expert * e, static_cast<double>(m) * topk);
 }

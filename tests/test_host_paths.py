@@ -3,6 +3,7 @@
 import os
 import subprocess
 import sys
+import time
 import types
 
 import pytest
@@ -121,3 +122,13 @@ def test_no_alloc_accepted_set(switch):
                        timeout=300)
     assert r.returncode == 0, r.stderr[-2000:]
     assert r.stdout.strip().splitlines()[-1] == str(want)
+
+
+def test_plan_time_of_long_calls():
+    """A plan's block estimate does not walk a long call's blocks one by one
+    (2^27 tokens on one expert: 0.25 s for these plans)."""
+    _capi.schedule(2, 128, 128, 1, 1)
+    t0 = time.perf_counter()
+    for _ in range(30):
+        assert "tiled" in _capi.schedule(2 ** 27, 128, 128, 1, 1)
+    assert time.perf_counter() - t0 < 0.05

@@ -165,6 +165,10 @@ __device__ __forceinline__ void tiled_tile(const GemmParams& p, const int rb_id,
   static_assert(RB >= 1 && CB >= 1 && KK >= 1, "wave tile");
   static_assert(!GEMM1 || CB % 2 == 0, "gate/up pairing");
   static_assert(128 % WCOLS == 0, "a wave's columns inside a 128-column block");
+  // GEMM2 outputs of an odd multiple of 128 columns end in a tile of half the
+  // columns where a tile spans more than 128 (the others carry no clamp: it
+  // cost the fp8 256x128 tile a spilled register)
+  constexpr bool PARTIAL = !GEMM1 && BNR > 128;
   static_assert(tiled_ring_bytes<DT, C, COMPACT>() <= 160 * 1024, "gfx950 LDS is 160 KiB");
   // a compact ring holds whole per-wave activation load groups
   static_assert(!COMPACT || C::BMA % (NLA * C::LR) == 0, "compact ring rows");
@@ -226,8 +230,9 @@ __device__ __forceinline__ void tiled_tile(const GemmParams& p, const int rb_id,
       const int ncol = tile_n * (BNR / 2) + wc * HALF + in % HALF;
       wrow = (in >= HALF ? p.n_out : 0) + ncol;
     } else {
+      wrow = static_cast<int64_t>(tile_n) * BNR + j;
       // (a last tile of half the columns: the other half reads the last row)
-      wrow = min(static_cast<int64_t>(tile_n) * BNR + j, p.n_out - 1);
+      if constexpr (PARTIAL) wrow = min(wrow, p.n_out - 1);
     }
     b_src[i] = p.w + (wbase + wrow) * row_bytes + chunk_pos<C>(j, lchunk) * 16;
   }
@@ -259,7 +264,8 @@ __device__ __forceinline__ void tiled_tile(const GemmParams& p, const int rb_id,
       if (slot < BM + (GEMM1 ? 2 : BNR / 128)) {
         const int b = slot - BM;
         wb = GEMM1 ? (b ? p.n_out / 128 : 0) + tile_n * (BNR / 2) / 128
-                   : min(static_cast<int64_t>(tile_n) * (BNR / 128) + b, p.n_out / 128 - 1);
+                   : static_cast<int64_t>(tile_n) * (BNR / 128) + b;
+        if constexpr (PARTIAL) wb = min(wb, p.n_out / 128 - 1);
       }
       sc_src = p.w_scale + (wblk0 + wb) * kblocks;
     }
@@ -400,10 +406,10 @@ __device__ __forceinline__ void tiled_tile(const GemmParams& p, const int rb_id,
   int nlive = 0;
 #pragma unroll
   for (int i = 0; i < RB; ++i) nlive += first_sid[i] < p.numel ? 1 : 0;
-  // GEMM2 outputs of an odd multiple of 128 columns end in a tile of half
-  // the columns: a wave whose columns lie past the output (its WCOLS divide
-  // 128: all of them or none) loads for the others but multiplies nothing
-  const bool no_cols = !GEMM1 && static_cast<int64_t>(tile_n) * BNR + wn * WCOLS >= p.n_out;
+  // in a tile of half the columns, a wave whose columns lie past the output
+  // (its WCOLS divide 128: all of them or none) loads for the others but
+  // multiplies nothing
+  const bool no_cols = PARTIAL && static_cast<int64_t>(tile_n) * BNR + wn * WCOLS >= p.n_out;
   if (no_cols) nlive = 0;
 
   Frag fa[2][RB], fb[2][CB];

@@ -407,13 +407,9 @@ __global__ __launch_bounds__(C::NW * 64, 1) void moe_gemm_wide_kernel(const Gemm
   };
 
   // Fragment reads: lane reads row (lane & 31) of a 32-row block, logical
-  // chunk 2*kk + (lane >> 5): the lane's offset f_off[kk] within a block,
-  // the wave's blocks at a_base (block i of the wave: tile rows
-  // (2i + wm) * 32) and b_base (uniform) of a slot.
-  const int fr = lane & 31;
-  int f_off[KK];
-#pragma unroll
-  for (int kk = 0; kk < KK; ++kk) f_off[kk] = fr * SK + wide_chunk<C>(fr, 2 * kk + (lane >> 5)) * 16;
+  // chunk 2*kk + (lane >> 5): the lane's offset f_off[kk] within a block
+  // (tile_body's), the wave's blocks at a_base (block i of the wave: tile
+  // rows (2i + wm) * 32) and b_base (uniform) of a slot.
   const int a_base = wm * 32 * SK;
   const int b_base = B_OFF + wn * WCOLS * SK;
 
@@ -491,6 +487,15 @@ __global__ __launch_bounds__(C::NW * 64, 1) void moe_gemm_wide_kernel(const Gemm
     constexpr int NLIVE = decltype(nlive_c)::value;
     Acc acc[RB][CB];
     Frag fa[2][RB], fb[2][CB];
+    // (from a copy of the lane that the compiler cannot see through: offsets
+    // shared by the instances stay live through one's epilogue into the
+    // next, and the GEMM1s spilled a register)
+    int f_lane = lane;
+    asm("" : "+v"(f_lane));
+    int f_off[KK];
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk)
+      f_off[kk] = (f_lane & 31) * SK + wide_chunk<C>(f_lane & 31, 2 * kk + (f_lane >> 5)) * 16;
 #pragma unroll
     for (int i = 0; i < RB; ++i)
 #pragma unroll

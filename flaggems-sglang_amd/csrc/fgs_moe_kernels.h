@@ -40,7 +40,6 @@ struct GemmParams {
   uint32_t topk_magic;
   int32_t topk_sh1, topk_sh2;
   int32_t weight_on_input;
-  int32_t row_blocks;     // row blocks of the launch (tiled kernels)
   int32_t group_m;        // row blocks per rasterization band (tiled; 0: off)
   int32_t group_n;        // column tiles per rasterization group (tiled)
   int32_t ksplit;         // GEMM2 k splits; > 1: out is fp32 [ksplit][numel][n_out]

@@ -959,7 +959,6 @@ static int launch_tiled(const GemmParams& p, int row_blocks, hipStream_t stream)
   constexpr int kCols = GEMM1 ? C::BNR / 2 : C::BNR;
   const int tiles_n = static_cast<int>((p.n_out + kCols - 1) / kCols);
   GemmParams q = p;
-  q.row_blocks = row_blocks;
   set_topk_magic(&q);
   q.group_m = group_m_choice(C::BM, p);
   q.group_n = group_n_choice();
@@ -1073,8 +1072,8 @@ static int launch_cfg(bool gemm1, const GemmParams& p, int row_blocks,
 void tiled_plan_request(int dt, int cfg, bool gemm1, const GemmParams& p, int row_blocks,
                         WidePlanReq* req) {
   *req = WidePlanReq{};
-  if (tiled_config_supported(dt, cfg) && row_blocks > 0 && cfg == 0 && p.shape == kTileByConfig && wide_choice() >= 1 &&
-      wide_supported(dt, gemm1, p))
+  if (tiled_config_supported(dt, cfg) && row_blocks > 0 && cfg == 0 &&
+      p.shape == kTileByConfig && wide_choice() >= 1 && wide_supported(dt, gemm1, p))
     wide_plan_request(gemm1, p, row_blocks, req);
 }
 

@@ -1065,7 +1065,6 @@ static int wide_col_tiles(bool gemm1, const GemmParams& p) {
 static void wide_launch_shape(bool gemm1, const GemmParams& p, int row_blocks, GemmParams* q,
                               int64_t* cap) {
   *q = p;
-  q->row_blocks = row_blocks;
   if (gemm1 || q->ksplit < 1) q->ksplit = 1;
   if (gemm1 || !q->tail_part) q->tail_split = 0;
   if (q->tail_split) q->ksplit = 1;

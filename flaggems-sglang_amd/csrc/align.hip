@@ -5,10 +5,11 @@
 // flattened expert ids (:134) and a per-expert histogram (:137-139). The
 // output is the block-padded, expert-grouped order the grouped GEMMs consume.
 //
-// moe_align_kernel (more experts than moe_align_mid_kernel's LDS takes, below
-// 4096 slots, or any number of slots without scratch memory): one workgroup of 16 wave64s (and, asked for tile plans, a
-// second that writes them). Wave w owns the contiguous slot segment
-// [w*seg, (w+1)*seg). Pass 1 counts ids per (wave, expert) in LDS; pass 2
+// moe_align_kernel (from 769 slots, where moe_align_mid_kernel's LDS does not
+// take the experts -- from 854, by the number of waves -- or, past 4096 slots,
+// where there is no scratch memory): one workgroup of 16 wave64s (and, asked
+// for tile plans, a second that writes them). Wave w owns the contiguous slot
+// segment [w*seg, (w+1)*seg). Pass 1 counts ids per (wave, expert) in LDS; pass 2
 // turns the counts into per-expert padded offsets plus per-wave offsets
 // inside each expert (exclusive over waves, so lower slots come first);
 // pass 3 walks each segment in slot order, 64 slots at a time, ranking each
@@ -316,7 +317,8 @@ __global__ __launch_bounds__(kAlignThreads) void moe_align_mid_kernel(
 }
 
 // ------------------------------------------------ multi-workgroup variant ---
-// For more slots than moe_align_mid_kernel takes: the ids are cut into chunks of kChunk consecutive slots.
+// For more slots than moe_align_mid_kernel takes: the ids are cut into chunks
+// of kChunk consecutive slots.
 // Kernel 1 counts each chunk's ids per expert (counts[c][e]). Kernel 2 runs
 // one workgroup per chunk: it sums the counts of every chunk (totals) and of
 // the chunks before its own (its per-expert base, so lower slots come
@@ -597,8 +599,8 @@ int launch_align(const int32_t* ids, int64_t numel, int num_experts,
     hipLaunchKernelGGL(moe_align_scatter_kernel, dim3(nchunks + (with_plans ? 1 : 0)),
                        dim3(kChunkThreads),
                        smem2, stream, ids, numel, num_experts, block_size, id_bits,
-                       scratch, sorted_ids, expert_ids, num_post_pad, max_padded, plan0, plan1, other,
-                       hist, slot_pos);
+                       scratch, sorted_ids, expert_ids, num_post_pad, max_padded, plan0, plan1,
+                       other, hist, slot_pos);
     rc = check_launch("moe_align_scatter_kernel");
     if (!rc && planned) *planned = plan0.plan || plan1.plan;
     return rc;

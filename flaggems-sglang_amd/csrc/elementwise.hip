@@ -179,8 +179,8 @@ __global__ __launch_bounds__(256) void moe_sum_partials_kernel(
 // System/6000 processor", IBM J. Res. Dev. 1990): x * inv is within two ulps,
 // one residual step brings it within one, and a second from there, with a
 // correctly rounded reciprocal, gives the rounded quotient (and, with x's
-// sign, its signed zero). Six FMA-rate instructions in place of a division's ten and its reciprocal; the
-// quantisers were bound by those. Exact where the residuals are: a quotient
+// sign, its signed zero). Six FMA-rate instructions in place of a division's
+// ten and its reciprocal; the quantisers were bound by those. Exact where the residuals are: a quotient
 // small enough for one to lose bits rounds to code 0 either way.
 __device__ __forceinline__ float quotient(float x, float scale, float inv) {
   float q = x * inv;

@@ -154,8 +154,8 @@ class ScatterIndx:
 def standard_topk_to_routing(topk_weights, topk_ids, n_expts_tot):
     """``(topk_weights, topk_ids)`` -> ``(RoutingData, GatherIndx,
     ScatterIndx)`` in the reference's routing format, computed on the GPU
-    (``fgs_moe_topk_to_routing``: the stable alignment kernel plus two small
-    kernels).
+    (``fgs_moe_topk_to_routing``: the stable alignment and one kernel after
+    it).
 
     The result is that of ``_standard_topk_to_triton_kernels``
     (ops/fused_moe.py:119-146): per-token ascending id sort carrying the

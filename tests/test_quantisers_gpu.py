@@ -115,3 +115,26 @@ def test_repeated_slots_of_a_routing_tuple(gpu, mode, flags):
     ref = fm.fused_moe(x, wts.w1, wts.w2, w, ids, _flags=flags, **wts.kwargs(mode))
     # (a token with an unnamed slot reads what the workspace held for it: here -1, dropped)
     assert torch.equal(out, ref)
+
+
+@pytest.mark.parametrize("M", [110, 450])
+@pytest.mark.parametrize("mode", ["fp8", "int8"])
+def test_rows_of_many_experts(gpu, mode, M):
+    """880 and 3600 slots of 1024 experts: the alignment for more experts than
+    the single-workgroup one's LDS takes records the padded rows. The bits of
+    the routing-tuple path (its own order kernel), slots dropped and outside."""
+    K, N, E, topk = 256, 256, 1024, 8
+    wts = testing.make_weights(K, N, E, mode, 0.05, device=gpu, seed=M)
+    x, w, ids = testing.make_tokens(M, K, E, topk, device=gpu, seed=M)
+    w, ids = (t.gather(1, ids.argsort(1)) for t in (w, ids))
+    ids[::3, -1] = -1
+    known = ids >= 0
+    key = torch.where(known, ids, torch.full_like(ids, E)).reshape(-1)
+    src = key.sort(stable=True).indices.int()
+    hist = torch.bincount(key, minlength=E + 1)[:E].int()
+    rd = fm.RoutingData(w.reshape(-1)[src.long()].float(), hist, E, topk)
+    qm = {"fp8": _capi.QMODE_FP8_BLOCK, "int8": _capi.QMODE_INT8_CHANNEL}[mode]
+    ref = fm._fused_routed(x, wts.w1, wts.w2, rd, fm.GatherIndx(src, src), qmode=qm,
+                           w1_scale=wts.w1_scale, w2_scale=wts.w2_scale)
+    ids[::3, -1] = torch.where(torch.arange(len(ids[::3]), device=gpu) % 2 == 0, -1, E).int()
+    assert torch.equal(fm.fused_moe(x, wts.w1, wts.w2, w, ids, **wts.kwargs(mode)), ref)

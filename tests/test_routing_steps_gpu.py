@@ -33,11 +33,14 @@ def test_gating_ranks(gpu, E, scoring):
 
 
 @pytest.mark.parametrize("M,k,E", [(0, 4, 65), (8, 8, 64), (9, 8, 65), (64, 4, 128),
-                                   (512, 8, 129), (513, 8, 256), (700, 6, 1022), (3, 1, 1)])
+                                   (512, 8, 129), (513, 8, 256), (700, 6, 1022), (3, 1, 1),
+                                   (110, 8, 1022), (450, 8, 1022)])
 def test_conversion_tables(gpu, M, k, E):
     """One, 64, 65, 4095.. slots and whole and partial waves of experts: the
-    single-wave, single- and many-workgroup alignments write the histogram,
-    the last workgroup of the finishing launch the tables. Ids on either side
+    single-wave, single- and many-workgroup alignments (and, at 880 and 3600
+    slots of 1022 experts, the one for more experts than the single-workgroup
+    one's LDS takes) write the histogram, the last workgroup of the finishing
+    launch the tables. Ids on either side
     of [0, E) sort behind the experts and count for none."""
     g = torch.Generator().manual_seed(M + E)
     ids = torch.stack([torch.randperm(E, generator=g)[:k] for _ in range(M)]).int() if M else \

@@ -11,18 +11,18 @@ from test_fused_moe_gpu import _bias_inputs
 
 pytestmark = pytest.mark.gpu
 
-# m, hidden, inter, experts, topk, mode, flags, what the schedule says
+# m, hidden, inter, experts, topk, mode, flags, the schedule (in full)
 SHAPES = [(1, 4096, 256, 8, 2, "bf16", 0, "direct_sum"),
           (1, 2048, 768, 16, 8, "bf16", 0, "direct_sum pair"),
-          (1, 2048, 128, 8, 3, "fp8", 0, "direct_sum pair"),
-          (1, 4096, 256, 8, 2, "int8", 0, "direct_sum"),
+          (1, 2048, 128, 8, 3, "fp8", 0, "direct_sum pair qfold"),
+          (1, 4096, 256, 8, 2, "int8", 0, "direct_sum qfold_a2"),
           (1, 512, 256, 8, 2, "bf16", 0, "direct"),
-          (7, 512, 256, 8, 8, "bf16", 0, "stream"),
-          (7, 640, 128, 8, 3, "bf16", 0, "stream"),
-          (9, 512, 256, 8, 2, "int8", 0, "stream"),
-          (300, 512, 256, 8, 1, "fp8", _capi.flag_tile(0), "tiled"),
-          (300, 512, 256, 8, 4, "int8", _capi.flag_tile(1), "tiled"),
-          (128, 4096, 2560, 8, 2, "bf16", 0, "ksplit2")]
+          (7, 512, 256, 8, 8, "bf16", 0, "stream mt=1"),
+          (7, 640, 128, 8, 3, "bf16", 0, "stream mt=1"),
+          (9, 512, 256, 8, 2, "int8", 0, "stream mt=1"),
+          (300, 512, 256, 8, 1, "fp8", _capi.flag_tile(0), "tiled cfg=0 cfg2=0"),
+          (300, 512, 256, 8, 4, "int8", _capi.flag_tile(1), "tiled cfg=1 cfg2=1"),
+          (128, 4096, 2560, 8, 2, "bf16", 0, "tiled cfg=1 cfg2=1 ksplit2=2")]
 
 
 @pytest.mark.parametrize("M,K,N,E,topk,mode,flags,sched", SHAPES)
@@ -35,7 +35,7 @@ def test_scaled_is_mul(gpu, M, K, N, E, topk, mode, flags, sched, bias):
     kw = wts.kwargs(mode)
     qm = {"bf16": _capi.QMODE_BF16, "fp8": _capi.QMODE_FP8_BLOCK,
           "int8": _capi.QMODE_INT8_CHANNEL}[mode]
-    assert sched in _capi.schedule(M, K, N, E, topk, qm, flags)
+    assert _capi.schedule(M, K, N, E, topk, qm, flags) == sched
 
     def run(scale):
         if bias:

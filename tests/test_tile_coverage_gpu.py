@@ -51,11 +51,12 @@ def _within_ulps(res, ref):
 
 # the split tail on half tiles (1 to 8 rounds of tiles, 40 stages of k) and a
 # k split of them
-@pytest.mark.parametrize("shape", [(2100, 4224, 3200, 8, 2), (128, 4224, 2560, 8, 2)])
-def test_odd_hidden_splits(gpu, shape):
+@pytest.mark.parametrize("shape,split", [((2100, 4224, 3200, 8, 2), "tail2"),
+                                         ((128, 4224, 2560, 8, 2), "ksplit2=2")])
+def test_odd_hidden_splits(gpu, shape, split):
     M, K, N, E, topk = shape
     sched = _capi.schedule(M, K, N, E, topk, _capi.QMODE_BF16)
-    assert "tail2" in sched or "ksplit2" in sched, sched
+    assert split in sched.split(), sched
     x, w1, w2, b1, b2, w, ids = _bias_inputs(M, K, N, E, topk, gpu)
     toks = _sample(M, 48)
     res = fm.fused_moe(x, w1, w2, w, ids)
@@ -119,23 +120,23 @@ _QM = {"bf16": _capi.QMODE_BF16, "fp8": _capi.QMODE_FP8_BLOCK, "int8": _capi.QMO
 _SCHEDULED = [
     # 128x128 tiles, one per CU: k rows of one or two stages, of less and of
     # more than the ring, the last block of an expert partly filled
-    ("bf16", (60, 128, 128, 4, 2), "deep1 deep2"),
-    ("bf16", (61, 384, 256, 4, 2), "deep1 deep2"),
-    ("bf16", (700, 1152, 640, 4, 2), "deep1 deep2"),
-    ("int8", (60, 256, 256, 4, 2), "deep1 deep2"),
-    ("int8", (500, 1280, 768, 4, 2), "deep1 deep2"),
-    ("fp8", (60, 128, 128, 4, 2), "deep1 deep2"),
-    ("fp8", (333, 896, 640, 4, 2), "deep1 deep2"),
+    ("bf16", (60, 128, 128, 4, 2), "cfg=1 cfg2=1 deep1 deep2"),
+    ("bf16", (61, 384, 256, 4, 2), "cfg=1 cfg2=1 deep1 deep2"),
+    ("bf16", (700, 1152, 640, 4, 2), "cfg=1 cfg2=1 deep1 deep2"),
+    ("int8", (60, 256, 256, 4, 2), "cfg=1 cfg2=1 deep1 deep2"),
+    ("int8", (500, 1280, 768, 4, 2), "cfg=1 cfg2=1 deep1 deep2"),
+    ("fp8", (60, 128, 128, 4, 2), "cfg=1 cfg2=1 deep1 deep2"),
+    ("fp8", (333, 896, 640, 4, 2), "cfg=1 cfg2=1 deep1 deep2"),
     # fp8 GEMM1 two workgroups per CU on halves of 256-row blocks
-    ("fp8", (1700, 128, 1024, 32, 4), "dual1"),
-    ("fp8", (1801, 384, 1152, 32, 4), "dual1"),
+    ("fp8", (1700, 128, 1024, 32, 4), "cfg=0 cfg2=1 dual1"),
+    ("fp8", (1801, 384, 1152, 32, 4), "cfg=0 cfg2=1 dual1"),
     # fp8 GEMM2 on the 160-row ring
-    ("fp8", (1050, 384, 2560, 16, 2), "cfg=0 cfg2=0"),
+    ("fp8", (1050, 384, 2560, 16, 2), "cfg=0 cfg2=0 ksplit2=2"),
     # the split tail, a k split
-    ("bf16", (2600, 1152, 2560, 32, 2), "tail2"),
-    ("int8", (2600, 1280, 5120, 32, 2), "tail2"),
-    ("bf16", (128, 4096, 4096, 8, 2), "cfg2=1 ksplit2=2"),
-    ("bf16", (128, 1280, 4096, 8, 2), "deep2 ksplit2=3"),
+    ("bf16", (2600, 1152, 2560, 32, 2), "cfg=0 cfg2=0 tail2"),
+    ("int8", (2600, 1280, 5120, 32, 2), "cfg=0 cfg2=0 tail2"),
+    ("bf16", (128, 4096, 4096, 8, 2), "cfg=1 cfg2=1 ksplit2=2"),
+    ("bf16", (128, 1280, 4096, 8, 2), "cfg=1 cfg2=1 deep2 ksplit2=3"),
 ]
 
 
@@ -146,7 +147,7 @@ def test_scheduled_shapes(gpu, mode, shape, expect):
     oracle and (tiled) bit for bit against the 128-row configuration."""
     M, K, N, E, topk = shape
     sched = _capi.schedule(M, K, N, E, topk, _QM[mode])
-    assert expect in sched, sched
+    assert sched == "tiled " + expect
     wts = testing.make_weights(K, N, E, mode, 0.05, device=gpu, seed=M + K + N)
     x, w, ids = testing.make_tokens(M, K, E, topk, device=gpu, seed=M + K + N)
     res = fm.fused_moe(x, wts.w1, wts.w2, w, ids, **wts.kwargs(mode))

@@ -221,36 +221,67 @@ static int pick_kw(int64_t kdim, int step, int cap, int min_steps) {
 }
 
 // Rows per expert up to which a call streams, by GEMM1's 128-column tiles
-// over the touched experts (`k_bytes`: GEMM2's k row). The tiled kernels'
-// pipeline pays off earlier the more tiles share its fill, and the small
-// grids have the 128x128 tiles. Layer time, streaming / tiled, over weights
-// rotated through more memory than the caches (rows per expert: ratio):
-// bf16 48 tiles 10: 1.01, 12: 1.04; 64 8: 0.96, 10: 1.05; 112 10: 0.99, 12:
-// 1.06; 128 10: 0.93, 12: 1.00; 768 (1.5 KiB k rows) 12: 0.93, 14: 1.10; 736
-// 8: 0.97, 10: 1.03; 896 8: 0.94, 10: 0.98, 12: 1.09; 1280 6: 0.97, 8:
-// 1.01; 1536 6: 0.93, 8: 0.99; 1920 6: 0.98, 8: 1.02; 2944 6: 1.00, 8:
-// 1.04. int8 48 tiles 12: 0.98, 14: 1.04; 112 12: 0.96, 14: 1.09; 128 12:
-// 0.95, 14: 1.06; 768 4: 1.00, 6: 1.03; 704 6: 0.98, 8: 0.99, 10: 1.03; 896
-// 6: 0.99, 8: 1.02; 1280 4: 1.00, 6: 1.07; 1536 4: 1.03; 1920 6: 1.00, 8:
-// 1.03; 2816 4: 1.07. fp8 48 tiles 8: 1.00, 14: 1.08; 112 4: 0.97, 8: 1.02;
-// 128 8: 0.95, 10: 1.02; 736 and more 4: 1.03 to 1.15.
+// over the touched experts. The tiled GEMM1 runs them in rounds of the CUs, so
+// just past a round (257 to 400 tiles, 513 to 640, 769 to 850) it leaves most
+// of them idle and streaming lasts longest, and with every further round it
+// ends earlier; up to 112 tiles are cut into 128x128 ones.
+// Measured: 20900 calls of 8 to 256 experts (hidden 1024 to 7168, intermediate
+// 256 to 14336, weights rotated through more memory than the caches), both
+// schedules in turn. On 5360 further calls the chosen one is within 0.4 % of
+// the better one in the geometric mean, and in 95 of 100 within 2 % (int8 4).
+// Layer time, streaming / tiled, over the two rows below / above the line:
+//   tiles    bf16         int8         fp8
+//     32  0.91 0.95    0.99 1.00    0.96 1.05
+//     64  0.97 1.00    0.97 1.05    0.98 1.01
+//    112  1.00 1.03    0.99 1.02         1.02
+//    128  0.95 1.06    0.98 1.10    0.97 1.04
+//    160  0.98 1.06    0.97 1.02    0.96 1.01
+//    256  0.98 1.04    0.99 1.01    0.96 1.03
+//    320  0.92 1.07    0.96 1.17    0.98 1.00
+//    400  0.97 1.13    0.96 1.01    0.98 1.02
+//    512  0.97 1.03    0.98 1.03    0.98 1.04
+//    640  0.97 1.10    0.98 1.03    0.97 1.00
+//    768  0.97 1.02    0.97 0.99         1.00
+//    850  0.97 1.08    0.93 1.02    0.99 1.03
+//   1024  0.96 1.01    0.95 1.00    0.93 1.02
+//   1110  0.97 1.05    0.94              1.03
+//   1300  0.97 1.02    0.98 1.01         1.03
+//   2000  0.98 1.02         1.04         1.07
+//   3000  0.99 1.03         1.07         1.12
+//   more       1.02         1.11         1.19
 //
-// A GEMM2 of at most 100 256-column tiles over the touched experts leaves the
-// tiled kernels most CUs idle even split over k, and streaming lasts longer.
-// Layer time, streaming / tiled, at 10 rows (16-row blocks) and 12.5 (32-row
-// blocks; 16-row ones are up to 13 % faster), hidden/intermediate/experts: bf16
-// 2048/8448/8 0.75, 0.98; 3072/8448/8 0.91, 1.14; 1280/4352/8 0.86, 1.04;
-// 2048/4352/8 0.72, 0.87; 3072/4352/8 0.83, 0.96; 1536/7168/16 0.99, 1.30.
-// int8 2048/8448/8 1.00, 1.32; 2048/4352/8 0.89, 1.12; 1536/7168/16 1.12;
-// fp8 2048/8448/8 1.04; 2048/4352/8 0.93, 1.16; 3072/4352/8 0.97, 1.16.
-static double stream_rows(int dt, double tiles, double tiles2, int64_t k_bytes) {
-  if (tiles2 <= 100 && tiles > 160) {
-    if (dt == kDtBf16 && tiles <= 1000) return tiles <= 400 ? 12.5 : 10.5;
-    if (tiles <= (dt == kDtInt8 ? 600 : 400)) return 10.5;
+// `hidden4k`, `inter4k`: a weight row of GEMM1 / GEMM2 is a multiple of 4 KiB.
+// The tiled kernels lose more to such a stride (256 rows of it in flight per
+// workgroup, likely on few memory channels) than the streaming ones (16): 5 to
+// 7 % of the layer for hidden, 4 to 5 % for the intermediate size, 10 to 25 %
+// for both. The lines move up, as far as 16-row blocks reach (bf16 past 640
+// tiles to 11.5: 1.14 at 12 rows with both). Layer time at 6 to 7 rows, 512 /
+// 1024 / 2000 tiles, both: bf16 0.65 / 0.74 / 0.81, int8 0.74 / 0.80 / 0.89,
+// fp8 (5 rows) 0.81 / 0.88 / 0.92. Distance of the chosen from the better one
+// without this and with it, bf16, fp8, int8: hidden 0.8, 1.6, 1.3 -> 0.4, 1.0,
+// 0.4 %; both 3.4, 7.2, 8.1 -> 0.7, 1.2, 0.2 %.
+static double stream_rows(int dt, double tiles, bool hidden4k, bool inter4k) {
+  static const struct {
+    double tiles, rows[3];  // up to so many tiles: rows of bf16, fp8, int8
+  } kLines[] = {
+      {32.5, {25, 12.5, 17}},    {64.5, {13.5, 9.5, 12.5}},  {112.5, {9.5, 2, 9}},
+      {128.5, {12.5, 8.5, 12}},  {160.5, {12, 5, 9.5}},      {256.5, {10, 2.5, 7}},
+      {320.5, {12.5, 9, 12.5}},  {400.5, {12, 4.5, 9}},      {512.5, {9.5, 2.5, 7}},
+      {640.5, {11.5, 4.5, 9.5}}, {768.5, {9.5, 2, 5.5}},     {850.5, {11, 3.5, 4}},
+      {1024.5, {9, 2.5, 5.5}},   {1110.5, {10, 2.5, 4}},     {1300, {8, 2, 4}},
+      {2000, {7.5, 2, 2}},       {3000, {6.5, 2, 2}},
+  };
+  static const double kStride[3][4] = {  // rows more: neither, hidden, inter, both
+      {0, 2.5, 2, 3}, {0, 1.5, 1, 6.5}, {0, 4.5, 0, 7}};
+  double line = dt == kDtBf16 ? 4.5 : 2;
+  for (const auto& l : kLines) {
+    if (tiles > l.tiles) continue;
+    line = l.rows[dt];
+    break;
   }
-  if (dt == kDtFp8) return tiles <= 160 ? 7 : 3;
-  if (dt == kDtInt8) return tiles <= 160 ? 12.5 : tiles <= 1000 ? 6 : tiles <= 2000 ? 4.5 : 3;
-  return tiles <= 160 ? 10 : tiles <= 1000 ? (k_bytes < 2048 ? 12.5 : 9) : tiles <= 2000 ? 7 : 5.5;
+  const double more = kStride[dt][(hidden4k ? 1 : 0) + (inter4k ? 2 : 0)];
+  const double reach = dt == kDtBf16 && tiles > 640.5 ? 11.5 : 12.5;
+  return std::max(line, std::min(line + more, reach));
 }
 
 // The schedule of a call with many rows: streaming or tiled, the tile
@@ -269,15 +300,14 @@ static void call_rule(int64_t m, int64_t hidden, int64_t inter, int e, int topk,
   // Streaming row blocks: 16 rows up to 12.5 rows per expert (8 experts,
   // hidden 1920, intermediate 4224, 12.5 rows: 106 us in blocks of 32, 93 of
   // 16; more would give a share of the experts a second block, which streams
-  // their weights again), 32 up to 28 (bf16 hidden 3584, intermediate 2560, 64 experts, 16
-  // rows: GEMM1 614 us in blocks of 16, 528 of 32), else 64.
+  // their weights again), 32 up to 28 (bf16 hidden 3584, intermediate 2560, 64
+  // experts, 16 rows: GEMM1 614 us in blocks of 16, 528 of 32), else 64.
   p.mt = rows <= 12.5 ? 1 : rows <= 28 ? 2 : 4;
   // Tiled kernels (deep DMA pipeline) or streaming ones (weights straight
   // into registers), by rows per expert: see stream_rows.
   const double touched = e * (1.0 - std::exp(-rows));
-  const double stream_to =
-      stream_rows(p.dt, touched * static_cast<double>(inter / 128),
-                  touched * static_cast<double>((hidden + 255) / 256), inter * esz);
+  const double stream_to = stream_rows(p.dt, touched * static_cast<double>(inter / 128),
+                                       hidden * esz % 4096 == 0, inter * esz % 4096 == 0);
   // One token always streams (its direct-row schedule). Every accepted shape
   // can run tiled: a hidden size that is an odd multiple of 128 ends GEMM2 in
   // a half tile. (Streaming reads an expert's weights once per block of at

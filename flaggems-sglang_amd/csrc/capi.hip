@@ -111,12 +111,16 @@ static double expected_blocks(int64_t m, int topk, int e, int bm) {
 // round costs more than it saves (measured at 256 rows per expert, one box:
 // fp8 hidden 1280, intermediate 3072, 64 experts GEMM2 and sum 260 us with
 // the split that filled the last round, 147 without; Mixtral's long rows at
-// 32 tokens per expert 246 us unsplit, 174 in two).
+// 32 tokens per expert 246 us unsplit, 174 in two). The split grid has to fit
+// one round (2 % for the estimate): 88 tiles in three, 264, take 114 us of
+// layer (hidden 2688, intermediate 3584, 8 experts, 23 rows), in two 98;
+// 136 in two 471 (hidden 4224, intermediate 11648), whole 424. Over 1024 drawn
+// calls with every split forced the choice is within 0.4 % of the best one.
 static int pick_ksplit(double tiles, int64_t stages, int64_t numel, int64_t hidden) {
   int best = 1;
   double best_gain = 0.0;
   for (int s = 2; s <= 4; ++s) {
-    if (stages < 8 * s || tiles * s > 1.1 * kNumCUs) break;
+    if (stages < 8 * s || tiles * s > 1.02 * kNumCUs) break;
     const double gain = 0.9 * static_cast<double>(stages) * (1.0 - 1.0 / s) - 3.0 -
                         static_cast<double>(numel) * static_cast<double>(hidden) * (8 * s - 4) / 4e6;
     if (gain > best_gain) {

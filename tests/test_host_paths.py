@@ -132,3 +132,15 @@ def test_plan_time_of_long_calls():
     for _ in range(30):
         assert "tiled" in _capi.schedule(2 ** 27, 128, 128, 1, 1)
     assert time.perf_counter() - t0 < 0.05
+
+
+@pytest.mark.parametrize("qmode,shape,split", [
+    (_capi.QMODE_BF16, (92, 2688, 3584, 8, 2), "ksplit2=2"),       # 88 tiles
+    (_capi.QMODE_FP8_BLOCK, (381, 1408, 13312, 8, 2), "ksplit2=2"),  # 88 of 128 columns
+    (_capi.QMODE_BF16, (83, 4224, 11648, 8, 2), ""),               # 136
+    (_capi.QMODE_BF16, (128, 1280, 4096, 8, 2), "ksplit2=3")])     # 80 of 128 columns
+def test_k_split_fits_one_round(qmode, shape, split):
+    """GEMM2's k split stays within one round of the 256 CUs: a few tiles past
+    it make a second round (88 tiles in three 16 % slower than in two)."""
+    sched = _capi.schedule(*shape, qmode)
+    assert [w for w in sched.split() if "split" in w] == split.split(), sched

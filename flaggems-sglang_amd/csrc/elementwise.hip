@@ -189,6 +189,15 @@ __device__ __forceinline__ float quotient(float x, float scale, float inv) {
   return __builtin_copysignf(q, x);
 }
 
+// The scale for quotient's residuals: itself, or zero for an infinite one (an
+// infinity in the row or group), with which a finite x gives its signed zero
+// and an infinity NaN, as the division does. (With a division as the other
+// branch, per value: int8, 20000 rows of 128 columns 10.2 us, 7.3 so, 1024 of
+// 8192 12.6 and 9.9, one of 14336 6.0 and 5.2; divisions alone 8.1, 11.4, 5.7.)
+__device__ __forceinline__ float residual_scale(float scale) {
+  return scale < INFINITY ? scale : 0.f;
+}
+
 // The row of x a quantiser's work item `i` takes: i, or the padded row given
 // for it (-1: none).
 __device__ __forceinline__ int64_t quant_row(const int32_t* row_of, int64_t i,
@@ -236,14 +245,9 @@ __global__ __launch_bounds__(256) void quant_fp8_group_kernel(
     amax = fmaxf(amax, __shfl_xor(amax, d, 64));
   if (!active) return;
   const float scale = fmaxf(amax, 1e-10f) / 448.0f;
-  if (scale < INFINITY) {
-    const float inv = 1.0f / scale;
+  const float inv = 1.0f / scale;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) f[j] = quotient(f[j], scale, inv);
-  } else {  // an infinity in the group
-#pragma unroll
-    for (int j = 0; j < 8; ++j) f[j] = f[j] / scale;
-  }
+  for (int j = 0; j < 8; ++j) f[j] = quotient(f[j], residual_scale(scale), inv);
   uint32_t lo = 0, hi = 0;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
@@ -301,14 +305,15 @@ __global__ __launch_bounds__(256) void moe_scale_gather_kernel(
 
 // ----------------------------------------------------- int8 token quant ---
 constexpr int64_t kInt8WaveRows = 1024;  // rows from which a wave takes a row
-// Eight values of a row -> int8 codes rne(x / scale) clamped to +-127.
+// Eight values of a row -> int8 codes rne(x / scale) clamped to +-127
+// (`scale`: residual_scale's).
 __device__ __forceinline__ uint2 quant_int8x8(const u32x4& w, float scale, float inv) {
   uint32_t packed[2] = {0, 0};
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
     const float f = (j & 1) ? __uint_as_float(w[j / 2] & 0xffff0000u)
                             : __uint_as_float(w[j / 2] << 16);
-    float rq = __builtin_rintf(scale < INFINITY ? quotient(f, scale, inv) : f / scale);
+    float rq = __builtin_rintf(quotient(f, scale, inv));
     rq = fminf(fmaxf(rq, -127.f), 127.f);
     const uint32_t b = static_cast<uint32_t>(static_cast<int32_t>(rq)) & 0xffu;
     packed[j / 4] |= b << (8 * (j & 3));
@@ -351,11 +356,11 @@ __global__ __launch_bounds__(256) void quant_int8_token_kernel(
 #pragma unroll
   for (int d = 32; d >= 1; d >>= 1) amax = fmaxf(amax, __shfl_xor(amax, d, 64));
   const float scale = fmaxf(amax, 1e-10f) / 127.0f;
-  const float inv = 1.0f / scale;
+  const float inv = 1.0f / scale, res = residual_scale(scale);
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
     const int64_t c = (static_cast<int64_t>(v) * 64 + lane) * 8;
-    if (c < cols) *reinterpret_cast<uint2*>(dst + c) = quant_int8x8(w[v], scale, inv);
+    if (c < cols) *reinterpret_cast<uint2*>(dst + c) = quant_int8x8(w[v], res, inv);
   }
   if (lane == 0) scales[r] = scale;
 }
@@ -445,10 +450,10 @@ __global__ __launch_bounds__(256) void quant_int8_token_wg_kernel(
   __syncthreads();
   amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
   const float scale = fmaxf(amax, 1e-10f) / 127.0f;
-  const float inv = 1.0f / scale;
+  const float inv = 1.0f / scale, res = residual_scale(scale);
   for (int64_t c = threadIdx.x * 8; c < cols; c += 256 * 8)
     *reinterpret_cast<uint2*>(dst + c) =
-        quant_int8x8(*reinterpret_cast<const u32x4*>(src + c), scale, inv);
+        quant_int8x8(*reinterpret_cast<const u32x4*>(src + c), res, inv);
   if (threadIdx.x == 0) scales[r] = scale;
 }
 

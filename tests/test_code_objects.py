@@ -1,5 +1,5 @@
-"""The built gfx950 code objects' metadata: no kernel that a call can reach by
-its own schedule keeps registers in scratch memory."""
+"""The built gfx950 code objects: no kernel that a call can reach by its own
+schedule keeps registers in scratch memory, and the quantisers' divisions."""
 
 import os
 import shutil
@@ -22,8 +22,14 @@ SPILLING = ("moe_gemm_tiled_kernelILi1ENS_7TileCfgILi160E",
             "moe_gemm_stream_kernelILi2ELi4ELi8ELb1ELb0ELb0E")
 
 
-def _kernels(lib, tmp):
-    """[(name, metadata)] of every kernel for gfx950 in the library."""
+LIB = os.path.join(os.path.dirname(_capi.__file__), _capi.LIB_NAME)
+pytestmark = pytest.mark.skipif(
+    not all(shutil.which(f"{LLVM}/{t}") for t in ("llvm-objcopy", "llvm-readelf", "llvm-objdump")),
+    reason="no LLVM object tools under /opt/rocm")
+
+
+def _objects(lib, tmp):
+    """The paths of the library's gfx950 code objects."""
     fat = os.path.join(tmp, "fat")
     subprocess.run([f"{LLVM}/llvm-objcopy", "--dump-section", f".hip_fatbin={fat}", lib,
                     os.path.join(tmp, "copy.so")], check=True, capture_output=True)
@@ -39,25 +45,42 @@ def _kernels(lib, tmp):
             p += 24 + length
             if "gfx950" not in triple or size == 0:
                 continue
-            obj = os.path.join(tmp, "obj")
-            with open(obj, "wb") as f:
+            out.append(os.path.join(tmp, f"obj{len(out)}"))
+            with open(out[-1], "wb") as f:
                 f.write(data[at + offset:at + offset + size])
-            notes = subprocess.run([f"{LLVM}/llvm-readelf", "--notes", obj], check=True,
-                                   capture_output=True, text=True).stdout
-            meta = notes[notes.index("---"):notes.index("...\n")]
-            kernels = yaml.safe_load(meta).get("amdhsa.kernels") or []
-            out += [(k[".name"], k) for k in kernels]
         at = data.find(MAGIC, at + 1)
     return out
 
 
-@pytest.mark.skipif(not all(shutil.which(f"{LLVM}/{t}") for t in ("llvm-objcopy", "llvm-readelf")),
-                    reason="no LLVM object tools under /opt/rocm")
+def _tool(name, *args):
+    return subprocess.run([f"{LLVM}/{name}", *args], check=True, capture_output=True,
+                          text=True).stdout
+
+
+def _kernels(obj):
+    """[(name, metadata)] of an object's kernels."""
+    notes = _tool("llvm-readelf", "--notes", obj)
+    meta = notes[notes.index("---"):notes.index("...\n")]
+    return [(k[".name"], k) for k in yaml.safe_load(meta).get("amdhsa.kernels") or []]
+
+
 def test_no_scratch_memory(tmp_path):
-    lib = os.path.join(os.path.dirname(_capi.__file__), _capi.LIB_NAME)
-    kernels = _kernels(lib, str(tmp_path))
+    kernels = [k for obj in _objects(LIB, str(tmp_path)) for k in _kernels(obj)]
     assert len(kernels) > 150
     spilled = {n: (k[".private_segment_fixed_size"], k[".vgpr_spill_count"]) for n, k in kernels
                if (k[".private_segment_fixed_size"] or k[".vgpr_spill_count"])
                and not any(s in n for s in SPILLING)}
     assert not spilled, spilled
+
+
+def test_quantisers_divide_per_row_only(tmp_path):
+    """The quantisers divide twice a row or group (its scale and the scale's
+    reciprocal) and not per value, infinities included."""
+    seen = set()
+    for obj in _objects(LIB, str(tmp_path)):
+        names = [n for n, _ in _kernels(obj) if "quant_int8_token" in n or "quant_fp8_group" in n]
+        for n in names:
+            code = _tool("llvm-objdump", "-d", f"--disassemble-symbols={n}", obj)
+            seen.add(n)
+            assert code.count("v_div_fixup_f32") <= 2, n
+    assert len(seen) > 10

@@ -73,6 +73,18 @@ def test_no_scratch_memory(tmp_path):
     assert not spilled, spilled
 
 
+def test_plain_sum_carries_no_output_scale(tmp_path):
+    """The unscaled sum of eight (or two) slots rounds its eight values once:
+    no second rounding behind a test of the output's scale."""
+    packs = {}
+    for obj in _objects(LIB, str(tmp_path)):
+        for n in (n for n, _ in _kernels(obj) if "moe_sum_tk_kernel" in n):
+            code = _tool("llvm-objdump", "-d", f"--disassemble-symbols={n}", obj)
+            packs[n] = code.count("v_cvt_pk_bf16_f32")
+    plain = [c for n, c in packs.items() if "Lb0E" in n]
+    assert len(plain) == 2 and all(c <= 4 for c in plain), packs
+
+
 def test_quantisers_divide_per_row_only(tmp_path):
     """The quantisers divide twice a row or group (its scale and the scale's
     reciprocal) and not per value, infinities included."""

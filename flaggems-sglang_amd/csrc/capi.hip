@@ -122,7 +122,8 @@ static int pick_ksplit(double tiles, int64_t stages, int64_t numel, int64_t hidd
   for (int s = 2; s <= 4; ++s) {
     if (stages < 8 * s || tiles * s > 1.02 * kNumCUs) break;
     const double gain = 0.9 * static_cast<double>(stages) * (1.0 - 1.0 / s) - 3.0 -
-                        static_cast<double>(numel) * static_cast<double>(hidden) * (8 * s - 4) / 4e6;
+                        static_cast<double>(numel) * static_cast<double>(hidden) * (8 * s - 4) /
+                            4e6;
     if (gain > best_gain) {
       best_gain = gain;
       best = s;

@@ -185,8 +185,9 @@ __global__ __launch_bounds__(256) void moe_sum_partials_kernel(
 // one residual step brings it within one, and a second from there, with a
 // correctly rounded reciprocal, gives the rounded quotient (and, with x's
 // sign, its signed zero). Six FMA-rate instructions in place of a division's
-// ten and its reciprocal; the quantisers were bound by those. Exact where the residuals are: a quotient
-// small enough for one to lose bits rounds to code 0 either way.
+// ten and its reciprocal; the quantisers were bound by those. Exact where the
+// residuals are: a quotient small enough for one to lose bits rounds to code 0
+// either way.
 __device__ __forceinline__ float quotient(float x, float scale, float inv) {
   float q = x * inv;
   q = __builtin_fmaf(__builtin_fmaf(-scale, q, x), inv, q);
